@@ -210,6 +210,14 @@ size_t partial_bytes(uint32_t m, uint32_t n, uint32_t k, int nw) {
 void choose_split_k(MfmaArgs &a, int bm, float *partial) {
     const uint32_t groups = a.k / 64;
     const bool prefill = bm > 16 && tuning().prefill_kernel != 1 && prefill_supported(a);
+    if (const uint32_t wide = prefill ? prefill_wide_split(a, kMaxSplitK) : 0) {
+        if (wide > 1) {
+            a.ksplit = wide;
+            a.groups_per_split = ((groups + wide - 1) / wide + 1) & ~1u;
+            a.partial = partial;
+        }
+        return;
+    }
     const uint32_t rows = prefill ? prefill_block_m(a.p[0].w2.qw != nullptr) : (uint32_t)bm_rows(bm);
     const uint32_t cols = prefill ? prefill_block_rows(a.p[0].w2.qw != nullptr) : (uint32_t)bn_of(bm, false);
     const uint32_t tiles = ((a.m + rows - 1) / rows) * ((a.p[0].w.n + cols - 1) / cols);
