@@ -311,7 +311,10 @@ int kr_moe_scan_scatter(const uint32_t *selected, uint32_t num_assign, uint32_t 
  * re-reads them per routed token).  The reference also rounds gate.x, up.x and
  * d_a to bf16; here they stay f32.
  * workspace: kr_q4_moe_workspace_bytes(tokens, topk, hidden, inter) bytes,
- * 16-byte aligned; calls sharing it must not overlap in time.
+ * 16-byte aligned; calls sharing it must not overlap in time.  (With more than
+ * 16 assignments its last part, tokens * topk * inter / 4 bytes, serves the
+ * grouped matrix products of prefill-sized routings; a workspace without that
+ * part is accepted and takes the kernel for few tokens per expert.)
  * Limits: experts <= 256; hidden and inter multiples of 128 and <= 2048;
  * scales and biases 4-byte aligned. */
 size_t kr_q4_moe_workspace_bytes(uint32_t tokens, uint32_t topk, uint32_t hidden, uint32_t inter);

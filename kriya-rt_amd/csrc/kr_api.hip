@@ -746,9 +746,20 @@ int kr_moe_scan_scatter(const uint32_t *selected, uint32_t num_assign, uint32_t 
                       "kr_moe_scan_scatter");
 }
 
-size_t kr_q4_moe_workspace_bytes(uint32_t tokens, uint32_t topk, uint32_t hidden, uint32_t inter) {
+// MoE workspace: h [assign, inter] bf16 (sorted order), d [assign, hidden] f32 (before the down projection:
+// the grouped kernels' x operand and its S units, tokens * hidden * 2.25 bytes), then h's S units for the
+// grouped kernels.  A workspace without that last part is accepted and takes the few-token kernel.
+static size_t moe_basic_bytes(uint32_t tokens, uint32_t topk, uint32_t hidden, uint32_t inter) {
     const size_t assign = (size_t)tokens * topk;
     return round_up(assign * inter * 2, 256) + round_up(assign * hidden * 4, 256);
+}
+static size_t moe_grouped_bytes(uint32_t tokens, uint32_t topk, uint32_t hidden, uint32_t inter) {
+    return moe_basic_bytes(tokens, topk, hidden, inter) + round_up((size_t)tokens * topk * (inter / 64) * 16, 256);
+}
+
+size_t kr_q4_moe_workspace_bytes(uint32_t tokens, uint32_t topk, uint32_t hidden, uint32_t inter) {
+    return (uint64_t)tokens * topk > kMoeGemvMaxAssign ? moe_grouped_bytes(tokens, topk, hidden, inter)
+                                                       : moe_basic_bytes(tokens, topk, hidden, inter);
 }
 
 namespace {
@@ -797,7 +808,7 @@ int check_moe_experts(const kr_q4_matrix *gate, const kr_q4_matrix *up, const kr
     if (!aligned(y, dtype_size(y_dtype) * 4)) return fail(KR_E_ALIGN, "y must be aligned to 4 elements");
     if (!aligned(weights, 4) || !aligned(offsets, 4) || !aligned(sorted_assign, 4))
         return fail(KR_E_ALIGN, "routing arrays must be 4-byte aligned");
-    const size_t need = kr_q4_moe_workspace_bytes(tokens, topk, hidden, inter);
+    const size_t need = moe_basic_bytes(tokens, topk, hidden, inter);
     if (!workspace || workspace_bytes < need)
         return fail(KR_E_WORKSPACE, "workspace of %zu bytes required, %zu given", need, workspace_bytes);
     if (!aligned(workspace, 16)) return fail(KR_E_ALIGN, "workspace must be 16-byte aligned");
@@ -809,8 +820,8 @@ int check_moe_experts(const kr_q4_matrix *gate, const kr_q4_matrix *up, const kr
 int run_moe_experts(const kr_q4_matrix *gate, const kr_q4_matrix *up, const kr_q4_matrix *down, uint32_t experts,
                     const uint16_t *x, uint32_t tokens, uint32_t topk, const float *weights,
                     const uint32_t *offsets, const uint32_t *sorted_assign, int activation, void *y, int y_dtype,
-                    int accumulate, void *workspace, uint32_t hidden, uint32_t inter, void *stream,
-                    const FusedRoute *fr) {
+                    int accumulate, void *workspace, size_t workspace_bytes, uint32_t hidden, uint32_t inter,
+                    void *stream, const FusedRoute *fr) {
     hipStream_t s = (hipStream_t)stream;
     const uint32_t assign = tokens * topk;
     uint16_t *h = (uint16_t *)workspace;                                              // [assign, inter] bf16, sorted order
@@ -873,6 +884,48 @@ int run_moe_experts(const kr_q4_matrix *gate, const kr_q4_matrix *up, const kr_q
                           "kr_q4_moe_experts (combine)");
     }
 
+    // Ten tokens per expert (were they even): the grouped products, whose operands need the workspace's last part.
+    // Below, the few-token kernel's 16-row tiles move fewer zero rows: 60 experts, top 4, 64 tokens 104 us against 134,
+    // 128 tokens 135 / 140, 160 tokens 150 / 144, 256 tokens 185 / 153, 1000 tokens 480 / 222; 16 experts of [512,
+    // 1024], 60 tokens 42 / 30.
+    if (assign / std::min(experts, assign) >= 10 && workspace_bytes >= moe_grouped_bytes(tokens, topk, hidden, inter) &&
+        grouped_fits(inter, hidden, tokens, experts, assign) && grouped_fits(hidden, inter, assign, experts, assign)) {
+        uint16_t *xp = (uint16_t *)d;  // until the down projection writes d
+        char *xsu = (char *)d + round_up((size_t)tokens * hidden * 2, 256);
+        u32x4 *hsu = (u32x4 *)((char *)workspace + moe_basic_bytes(tokens, topk, hidden, inter));
+        if (hipError_t e = launch_moe_x_prep(x, tokens, hidden, xp, xsu, s)) return hip_status(e, "kr_q4_moe_experts (x)");
+        GroupedArgs gg{};
+        gg.w = to_mat(gate);
+        gg.w2 = to_mat(up);
+        gg.rows = inter;
+        gg.k = hidden;
+        gg.xp = xp;
+        gg.su = xsu;
+        gg.xrows = tokens;
+        gg.x_div = topk;
+        gg.offsets = offsets;
+        gg.sorted = sorted_assign;
+        gg.experts = experts;
+        gg.assign = assign;
+        gg.act = activation;
+        gg.out_h = h;
+        gg.out_su = hsu;
+        if (hipError_t e = launch_grouped(gg, s)) return hip_status(e, "kr_q4_moe_experts (gate/up)");
+        GroupedArgs gd = gg;
+        gd.w = to_mat(down);
+        gd.w2 = Q4Mat{};
+        gd.rows = hidden;
+        gd.k = inter;
+        gd.xp = h;
+        gd.su = hsu;
+        gd.xrows = assign;
+        gd.x_div = 0;
+        gd.out_d = d;
+        if (hipError_t e = launch_grouped(gd, s)) return hip_status(e, "kr_q4_moe_experts (down)");
+        return hip_status(launch_moe_combine(d, weights, tokens, topk, hidden, y, y_dtype == KR_DTYPE_F32, accumulate, s),
+                          "kr_q4_moe_experts (combine)");
+    }
+
     SkinnyArgs g{};
     g.w = to_mat(gate);
     g.w2 = to_mat(up);
@@ -921,7 +974,7 @@ int kr_q4_moe_experts(const kr_q4_matrix *gate, const kr_q4_matrix *up, const kr
         return rc;
     if (tokens == 0) return ok();
     return run_moe_experts(gate, up, down, experts, x, tokens, topk, weights, offsets, sorted_assign, activation, y,
-                           y_dtype, accumulate, workspace, hidden, inter, stream, nullptr);
+                           y_dtype, accumulate, workspace, workspace_bytes, hidden, inter, stream, nullptr);
 }
 
 int kr_q4_moe_route_experts(const kr_q4_matrix *gate, const kr_q4_matrix *up, const kr_q4_matrix *down,
@@ -949,21 +1002,21 @@ int kr_q4_moe_route_experts(const kr_q4_matrix *gate, const kr_q4_matrix *up, co
         moe_gemv_route_fits(experts, topk)) {
         const FusedRoute fr{logits, normalize, selected, counts};
         return run_moe_experts(gate, up, down, experts, x, tokens, topk, weights, offsets, sorted_assign, activation,
-                               y, y_dtype, accumulate, workspace, hidden, inter, stream, &fr);
+                               y, y_dtype, accumulate, workspace, workspace_bytes, hidden, inter, stream, &fr);
     }
     if (int rc = kr_moe_route(logits, tokens, experts, topk, normalize, selected, weights, counts, offsets,
                               sorted_assign, stream))
         return rc;
     if (tokens == 0) return ok();
     return run_moe_experts(gate, up, down, experts, x, tokens, topk, weights, offsets, sorted_assign, activation, y,
-                           y_dtype, accumulate, workspace, hidden, inter, stream, nullptr);
+                           y_dtype, accumulate, workspace, workspace_bytes, hidden, inter, stream, nullptr);
 }
 
 // kr_q4_moe_block workspace: router logits f32 [T, E], selected u32 [T*K], weights f32 [T*K],
 // counts u32 [E], offsets u32 [E+1], sorted u32 [T*K], then the experts' workspace.
 namespace {
 struct MoeBlockLayout {
-    size_t logits, selected, weights, counts, offsets, sorted, experts, total;
+    size_t logits, selected, weights, counts, offsets, sorted, experts, total, least;
 };
 MoeBlockLayout moe_block_layout(uint32_t tokens, uint32_t experts, uint32_t topk, uint32_t hidden, uint32_t inter) {
     const size_t assign = (size_t)tokens * topk;
@@ -977,6 +1030,7 @@ MoeBlockLayout moe_block_layout(uint32_t tokens, uint32_t experts, uint32_t topk
     L.sorted = o;   o += round_up(std::max<size_t>(assign, 1) * 4, 256);
     L.experts = o;  o += kr_q4_moe_workspace_bytes(tokens, topk, hidden, inter);
     L.total = o;
+    L.least = L.experts + moe_basic_bytes(tokens, topk, hidden, inter);
     return L;
 }
 }  // namespace
@@ -1020,8 +1074,8 @@ int kr_q4_moe_block(const kr_q4_matrix *router, const kr_q4_matrix *gate, const 
     if (!aligned(x, 16)) return fail(KR_E_ALIGN, "x must be 16-byte aligned");
     if (!aligned(y, dtype_size(y_dtype) * 4)) return fail(KR_E_ALIGN, "y must be aligned to 4 elements");
     const MoeBlockLayout L = moe_block_layout(tokens, experts, topk, hidden, inter);
-    if (!workspace || workspace_bytes < L.total)
-        return fail(KR_E_WORKSPACE, "workspace of %zu bytes required, %zu given", L.total, workspace_bytes);
+    if (!workspace || workspace_bytes < L.least)
+        return fail(KR_E_WORKSPACE, "workspace of %zu bytes required, %zu given", L.least, workspace_bytes);
     if (!aligned(workspace, 16)) return fail(KR_E_ALIGN, "workspace must be 16-byte aligned");
     char *ws = (char *)workspace;
     float *logits = (float *)(ws + L.logits);
@@ -1035,7 +1089,7 @@ int kr_q4_moe_block(const kr_q4_matrix *router, const kr_q4_matrix *gate, const 
     // down) and the weighted combine into y
     return kr_q4_moe_route_experts(gate, up, down, experts, x, tokens, topk, logits, normalize, selected, weights,
                                    counts, offsets, sorted, activation, y, y_dtype, accumulate, ws + L.experts,
-                                   L.total - L.experts, stream);
+                                   workspace_bytes - L.experts, stream);
 }
 
 int kr_q4_embedding(const kr_q4_matrix *w, const uint32_t *tokens, uint32_t count, uint16_t *out, void *stream) {

@@ -221,6 +221,25 @@ hipError_t launch_moe_gemv(MoeGemvArgs &a, int epilogue, hipStream_t s);
 // True when launch_moe_gemv can route the (single) token inside the gate/up launch.
 bool moe_gemv_route_fits(uint32_t experts, uint32_t topk);
 
+// ---- routed experts as grouped matrix products (q4_grouped.hip)
+struct GroupedArgs {
+    Q4Mat w, w2;              // stacked experts (w2: up matrix of the gate/up product, else qw == nullptr)
+    uint32_t rows, k;         // rows per expert, columns
+    const void *xp;           // bf16 [xrows, k], columns in pair order (launch_moe_x_prep)
+    const void *su;           // S units [xrows, k / 64], 16 bytes each
+    uint32_t xrows;
+    uint32_t x_div;           // > 0: X row of sorted position p is sorted[p] / x_div; 0: row p
+    const uint32_t *offsets, *sorted;
+    uint32_t experts, assign;
+    int act;
+    uint16_t *out_h;          // gate/up: bf16 [assign, rows] in sorted order, columns in pair order,
+    u32x4 *out_su;            //   and its S units [assign, rows / 64]
+    float *out_d;             // plain: f32 [assign, rows] in assignment order
+};
+hipError_t launch_moe_x_prep(const uint16_t *x, uint32_t rows, uint32_t k, void *xp, void *su, hipStream_t s);
+bool grouped_fits(uint32_t rows, uint32_t k, uint32_t xrows, uint32_t experts, uint32_t assign);
+hipError_t launch_grouped(const GroupedArgs &a, hipStream_t s);
+
 // ---- MoE routing and combine (moe.hip)
 constexpr uint32_t kRouteMaxTopK = 16;      // top-k list length of the routing kernel
 constexpr uint32_t kRouteMaxAssign = 16384; // T * K held in the routing block's LDS

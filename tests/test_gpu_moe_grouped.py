@@ -1,0 +1,118 @@
+"""GPU parity of the grouped expert products (csrc/q4_grouped.hip) and of the many-assignment routing scan against
+the CPU oracle: expert buckets at and around the tile heights (32 and 96 tokens), empty experts, odd numbers of
+128-column steps, every activation and output form, and a workspace without the grouped kernels' part.
+
+Bar: max |gpu - oracle| <= 1e-2 * RMS(oracle); routing integers exact.
+"""
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+from _util import assert_bf16_rounded_close, assert_rms_close, dev_bf16, host_bits, q4_dev, rms
+
+pytestmark = pytest.mark.gpu
+
+
+def synth():
+    from kriya_q4 import synth as s
+    return s
+
+
+def case(msg):
+    print(f"[case] {msg}", flush=True)
+
+
+def bucketed(counts, E):
+    """Expert ids [T, 1] that give the experts these bucket sizes, interleaved."""
+    ids = np.concatenate([np.full(n, e, np.uint32) for e, n in enumerate(counts)])
+    return np.random.default_rng(7).permutation(ids)[:, None]
+
+
+def setup(kq, ids, E, hidden, inter, seed):
+    s = synth()
+    T, K = ids.shape
+    g, u, d = (s.q4_weight(E * inter, hidden, seed), s.q4_weight(E * inter, hidden, seed + 1),
+               s.q4_weight(E * hidden, inter, seed + 2))
+    x = s.bf16_normal((T, hidden), seed + 3)
+    w = np.abs(s.f32_normal((T, K), seed + 4)) + 0.1
+    r = kq.MoeRoute(T, E, K)
+    sel = torch.from_numpy(np.ascontiguousarray(ids).view(np.int32)).cuda()
+    r.selected.copy_(sel)
+    r.weights.copy_(torch.from_numpy(w).cuda())
+    r.counts, r.offsets, r.sorted_assign = kq.moe_scan_scatter(sel.view(-1), E)
+    return (g, u, d), x, w, r
+
+
+@pytest.mark.parametrize("counts,hidden,inter,act", [
+    ((96, 97, 0, 95, 1, 64, 65, 193), 256, 128, 0),   # 96-token tiles: full, one over, one to three fragments
+    ((10, 0, 31, 32, 33, 1, 20, 30), 384, 640, 1),    # 32-token tiles; three and five steps
+    ((200, 0, 7), 128, 128, 2),                       # one step
+    ((41, 40, 39, 60), 2048, 1408, 0),
+])
+def test_buckets(kq, counts, hidden, inter, act):
+    E = len(counts)
+    case(f"grouped experts counts={counts} hidden={hidden} inter={inter} activation={act}")
+    ids = bucketed(counts, E)
+    (g, u, d), x, w, r = setup(kq, ids, E, hidden, inter, 6000)
+    want = O.moe_experts(O.Q4Planar(*g), O.Q4Planar(*u), O.Q4Planar(*d), E, x, ids, w, act)
+    G, U, D = q4_dev(kq, g), q4_dev(kq, u), q4_dev(kq, d)
+    T = ids.shape[0]
+    ws = kq.moe_workspace(T, 1, hidden, inter)
+    y = kq.moe_experts(G, U, D, E, dev_bf16(x), r, activation=act, workspace=ws).cpu().numpy()
+    for t in range(T):
+        assert_rms_close(y[t], want[t], what=f"token {t}")
+    y0 = synth().bf16_normal((T, hidden), 6100)
+    yb = dev_bf16(y0).clone()
+    kq.moe_experts(G, U, D, E, dev_bf16(x), r, y=yb, accumulate=True, activation=act, workspace=ws)
+    assert_bf16_rounded_close(host_bits(yb), O.bf16_to_f32(y0) + want, rms(want), rel=1e-2, what="bf16 accumulate")
+    # a workspace without the last part: the few-token kernel, the same values up to f32 summation order and the
+    # bf16 rounding of the intermediate
+    least = -(-T * inter * 2 // 256) * 256 + -(-T * hidden * 4 // 256) * 256
+    assert least < ws.numel()
+    z = kq.moe_experts(G, U, D, E, dev_bf16(x), r, activation=act, workspace=ws[:least]).cpu().numpy()
+    assert_rms_close(z, y, what="few-token kernel")
+
+
+def test_topk_rows_and_determinism(kq):
+    """Top-3 routing from logits (rows gathered through the sorted list), twice the same bits."""
+    case("grouped experts T=70 E=8 K=3")
+    s = synth()
+    T, E, K, hidden, inter = 70, 8, 3, 256, 256
+    g, u, d = s.q4_weight(E * inter, hidden, 6201), s.q4_weight(E * inter, hidden, 6202), s.q4_weight(E * hidden, inter, 6203)
+    x, logits = s.bf16_normal((T, hidden), 6204), s.f32_normal((T, E), 6205)
+    route = O.moe_route(logits, K, True)
+    want = O.moe_experts(O.Q4Planar(*g), O.Q4Planar(*u), O.Q4Planar(*d), E, x, route[0], route[1])
+    G, U, D = q4_dev(kq, g), q4_dev(kq, u), q4_dev(kq, d)
+    ys = [kq.moe_route_experts(G, U, D, E, dev_bf16(x), torch.from_numpy(logits).cuda(), K)[0].cpu().numpy()
+          for _ in range(2)]
+    assert_rms_close(ys[0], want, what="f32")
+    assert np.array_equal(ys[0].view(np.uint32), ys[1].view(np.uint32))
+
+
+def test_large_x_exact(kq):
+    """bf16 x far outside fp16's range stays exact (no fp16 operands here)."""
+    case("grouped experts, activations of 1e-6 and 1e6")
+    counts = (50, 40)
+    ids = bucketed(counts, 2)
+    (g, u, d), x, w, r = setup(kq, ids, 2, 256, 128, 6300)
+    xs = O.bf16_to_f32(x).copy()
+    xs[::2] *= 1e6
+    xs[1::2] *= 1e-6
+    x = O.f32_to_bf16(xs)
+    want = O.moe_experts(O.Q4Planar(*g), O.Q4Planar(*u), O.Q4Planar(*d), 2, x, ids, w, 0)
+    y = kq.moe_experts(q4_dev(kq, g), q4_dev(kq, u), q4_dev(kq, d), 2, dev_bf16(x), r).cpu().numpy()
+    for t in range(len(ids)):
+        assert_rms_close(y[t], want[t], what=f"token {t}")
+
+
+@pytest.mark.parametrize("n,E", [(257, 1), (1000, 3), (1025, 256), (4099, 60), (16384, 8)])
+def test_scan_scatter_many(kq, n, E):
+    """More assignments than one pass takes: parts per wave; ids >= E join no bucket."""
+    case(f"scan/scatter n={n} E={E}")
+    ids = np.random.default_rng(n).integers(0, E + 1, n).astype(np.uint32)
+    counts, offsets, scatter = kq.moe_scan_scatter(torch.from_numpy(ids.view(np.int32)).cuda(), E)
+    want = np.concatenate([np.nonzero(ids == e)[0] for e in range(E)])
+    assert np.array_equal(counts.cpu().numpy(), np.bincount(ids, minlength=E + 1)[:E])
+    assert int(offsets[-1]) == want.size
+    assert np.array_equal(scatter.cpu().numpy()[: want.size], want)
