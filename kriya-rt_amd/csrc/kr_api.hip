@@ -100,9 +100,8 @@ MfmaProblem problem(const Q4Mat &w, const Q4Mat *w2, void *out, const uint16_t *
     return p;
 }
 
-// Few-token matmul on the skinny kernel.  `partial` (f32 [ksplit, m, nw * n])
-// is needed when the K split exceeds one block; without it the caller must use
-// another path (returns hipErrorInvalidValue).  `tickets` (kSkinnyTickets zero
+// Few-token matmul on the skinny kernel.  With `partial` (f32 [ksplit, m, nw * n]) a K of more
+// than one slab is split over blocks; without it every block takes all slabs of its tiles.  `tickets` (kSkinnyTickets zero
 // words, left zero): the split is reduced inside the launch, else by a second one.
 // More than one launch's rows (32, or 16 with KR_OPT_SKINNY_GROUPS = 1; up to kSkinnyChunkMaxM):
 // chunks, one launch each, in row order; each reuses the partials and leaves the tickets at zero
@@ -111,7 +110,8 @@ hipError_t run_skinny(const Q4Mat &w, const Q4Mat *w2, const uint16_t *x, uint32
                       const uint16_t *bias, uint32_t ldo, int out_dtype, int accumulate, int act, float *partial,
                       hipStream_t s, const uint16_t *ln_w = nullptr, float eps = 0.0f,
                       uint32_t *tickets = nullptr) {
-    if (const uint32_t chunk = skinny_chunk_rows(); m > chunk) {
+    const bool loop = !partial && skinny_ksplit(w.k) > 1;  // one launch for any number of rows
+    if (const uint32_t chunk = skinny_chunk_rows(); m > chunk && !loop) {
         const size_t esz = dtype_size(out_dtype);
         for (uint32_t i0 = 0; i0 < m; i0 += chunk) {
             const uint32_t mc = std::min(chunk, m - i0);
@@ -137,13 +137,12 @@ hipError_t run_skinny(const Q4Mat &w, const Q4Mat *w2, const uint16_t *x, uint32
     a.out_f32 = out_dtype == KR_DTYPE_F32;
     a.accumulate = accumulate;
     const uint32_t ks = skinny_ksplit(w.k);
-    if (ks > 1) {
-        if (!partial) return hipErrorInvalidValue;
+    if (ks > 1 && partial) {
         a.partial = partial;
         if (tickets && tuning().splitk_tickets && ks <= kSkinnyMaxTicketSplit) a.tickets = tickets;
     }
     hipError_t e = launch_skinny(a, s);
-    if (e != hipSuccess || ks == 1 || a.tickets) return e;
+    if (e != hipSuccess || !a.partial || a.tickets) return e;
     MfmaArgs r{};
     r.p[0].w = w;
     r.p[0].out = out;
@@ -163,7 +162,7 @@ hipError_t run_skinny(const Q4Mat &w, const Q4Mat *w2, const uint16_t *x, uint32
 hipError_t run_skinny_qkv(const kr_q4_matrix *const *mats, const uint16_t *const *biases, void *const *outs,
                           const uint16_t *x, uint32_t m, int out_dtype, const uint16_t *ln_w, float eps,
                           hipStream_t s) {
-    if (const uint32_t chunk = skinny_chunk_rows(); m > chunk) {  // chunks, as run_skinny
+    if (const uint32_t chunk = skinny_chunk_rows(); m > chunk && skinny_ksplit(mats[0]->k) == 1) {  // chunks, as run_skinny
         const size_t esz = dtype_size(out_dtype);
         for (uint32_t i0 = 0; i0 < m; i0 += chunk) {
             void *o[3];
@@ -196,6 +195,20 @@ hipError_t run_skinny_qkv(const kr_q4_matrix *const *mats, const uint16_t *const
 // fp16, as the reference's M >= 64 kernels stage half.
 bool skinny_fits(uint32_t m, const Q4Mat &w, bool have_partial) {
     return m >= 2 && m <= kSkinnyChunkMaxM && skinny_supported(w) && (have_partial || skinny_ksplit(w.k) == 1);
+}
+
+// The same kernel over a K of several slabs without room for partials (its slab loop), `rows` weight rows in
+// all.  Before / with it, us: gate/up [2 x 9536, 3072], m = 2 .. 16 67-70 / 17, m = 32 41 / 22, m = 40 41 / 39;
+// q/k/v [4608, 3584], m = 2 45 / 10; linear [3584, 18944], m = 8 255 / 28, m = 32 77 / 39; [2048, 11008], m = 27
+// 46 / 18, m = 63 46 / 24; [16384, 2304], m = 24 16 / 20; [65536, 4096], m = 32 79 / 54.  So: gate/up up to 32
+// tokens; other launches up to 16 (kr_q4_linear: beyond k = 16384, the token GEMV's limit), and above where it is estimated faster (past 32 clearly so) than the prefill
+// kernels' 64-token tiles, whose time is about 4 us + 1.02 per 256 columns for every 16384 rows.
+bool skinny_loops(uint32_t m, const Q4Mat &w, uint32_t rows, bool gate_up) {
+    if (m < 2 || m > kSkinnyChunkMaxM || !skinny_supported(w) || skinny_ksplit(w.k) == 1) return false;
+    if (m <= (gate_up ? 32u : 16u)) return true;
+    if (gate_up) return false;
+    const float prefill = (4.0f + 0.004f * (float)w.k) * std::max(1.0f, (float)rows / 16384.0f);
+    return skinny_loop_us(m, rows, w.k, false) < (m <= 32 ? 1.0f : 0.8f) * prefill;
 }
 
 size_t partial_bytes(uint32_t m, uint32_t n, uint32_t k, int nw) {
@@ -471,7 +484,8 @@ int kr_q4_linear(const kr_q4_matrix *w, const uint16_t *x, uint32_t m, void *y, 
         // A few tokens over a K the few-token kernel needs a split-K workspace for (none here): the
         // token GEMV in chunks of up to kGemvMaxTokens tokens, every weight row read once per chunk
         // (m = 16, K = 11008: 36 us against 145 us for the unsplit tiled kernel).  Each token's row is
-        // the one a call with that token alone gives.
+        // the one a call with that token alone gives, bit for bit, which is why the slab loop (17 us, and
+        // 14 against 88 at [11008, 4096]) does not take these.
         const int epi = accumulate ? (y_dtype == KR_DTYPE_F32 ? kAccF32 : kAccBF16)
                                    : (y_dtype == KR_DTYPE_F32 ? kStoreF32 : kStoreBF16);
         const size_t ysz = dtype_size(y_dtype);
@@ -485,6 +499,9 @@ int kr_q4_linear(const kr_q4_matrix *w, const uint16_t *x, uint32_t m, void *y, 
         }
         return ok();
     }
+    if (skinny_loops(m, a, w->n, false))
+        return hip_status(run_skinny(a, nullptr, x, m, y, nullptr, w->n, y_dtype, accumulate, 0, nullptr, s),
+                          "kr_q4_linear");
     MfmaArgs args = mfma_args(x, m, w->k, y_dtype, accumulate);
     args.p[0] = problem(a, nullptr, y, nullptr, w->n);
     args.np = 1;
@@ -522,7 +539,7 @@ int kr_q4_gate_up_act(const kr_q4_matrix *gate, const kr_q4_matrix *up, const ui
         return hip_status(launch_gemv_tokens(g, &u, x, m, act_out, gate->n, epi, activation, nullptr, s),
                           "kr_q4_gate_up_act");
     }
-    if (skinny_fits(m, to_mat(gate), false) && skinny_supported(to_mat(up)))
+    if ((skinny_fits(m, g, false) || skinny_loops(m, g, gate->n, true)) && skinny_supported(u))
         return hip_status(run_skinny(g, &u, x, m, act_out, nullptr, gate->n, act_dtype, 0, activation, nullptr, s),
                           "kr_q4_gate_up_act");
     MfmaArgs args = mfma_args(x, m, gate->k, act_dtype, 0);
@@ -564,7 +581,8 @@ int kr_q4_qkv(const kr_q4_matrix *q, const kr_q4_matrix *k, const kr_q4_matrix *
         }
         return ok();
     }
-    if (skinny_fits(m, to_mat(q), false) && skinny_supported(to_mat(k)) && skinny_supported(to_mat(v)))
+    if ((skinny_fits(m, to_mat(q), false) || skinny_loops(m, to_mat(q), q->n + k->n + v->n, false)) && skinny_supported(to_mat(k)) &&
+        skinny_supported(to_mat(v)))
         return hip_status(run_skinny_qkv(mats, biases, outs, x, m, out_dtype, nullptr, 0.0f, s), "kr_q4_qkv");
     MfmaArgs args = mfma_args(x, m, q->k, out_dtype, 0);
     for (int i = 0; i < 3; ++i) args.p[i] = problem(to_mat(mats[i]), nullptr, outs[i], biases[i], mats[i]->n);

@@ -62,6 +62,7 @@ namespace {
 constexpr int kSkinnyWaves = 8;
 constexpr int kSkinnyPieces = 2;                                // 128-column pieces per wave
 constexpr int kSlabCols = kSkinnyWaves * kSkinnyPieces * 128;  // K columns per block
+constexpr uint32_t kLoopTiles = 16;                            // tiles a slab-loop block sums at a time
 
 __device__ __forceinline__ uint32_t opq_s(uint32_t v) {
     uint32_t r;
@@ -84,6 +85,14 @@ __device__ __forceinline__ u32x4 x_unit(const u32x4 &v) {
 __device__ __forceinline__ bf16x8_t q_frag(uint32_t w, uint32_t mask, uint32_t magic) {
     const u32x4 r = {(w & mask) | magic, ((w >> 4) & mask) | magic, ((w >> 8) & mask) | magic,
                      ((w >> 12) & mask) | magic};
+    return __builtin_bit_cast(bf16x8_t, r);
+}
+
+// The same with B = 16 + q: the nibble in mantissa bits 3 .. 6 under the bf16 pattern 0x4180 (one more shift).  The
+// group sum then cancels 16 S instead of 128 S, and the f32 roundings are about a fifth.
+__device__ __forceinline__ bf16x8_t q_frag16(uint32_t w, uint32_t mask, uint32_t magic) {
+    const u32x4 r = {((w << 3) & mask) | magic, ((w >> 1) & mask) | magic, ((w >> 5) & mask) | magic,
+                     ((w >> 9) & mask) | magic};
     return __builtin_bit_cast(bf16x8_t, r);
 }
 
@@ -116,7 +125,10 @@ __device__ __forceinline__ uint32_t xs_index(uint32_t r, uint32_t u) {
 // holds one group.  Its other half re-reads the live half's words (in the row, never past it), meets
 // zero X and a zero scale and bias, and the scale/bias pairs come in two 2-byte loads (a row's pairs
 // are not 4-byte aligned when K / 64 is odd).
-template <bool kGateUp, bool kGrouped, int MG, bool kPre, int D, bool kOdd>
+// kLoop: K longer than one slab with no room for partials (dense mode): a block takes every slab of its tiles in
+// turn, restaging X per slab, and keeps the sums over the slabs so far in LDS (one float per thread and tile, up
+// to kLoopTiles tiles at a time), added in slab order as the split-K reduction does.
+template <bool kGateUp, bool kGrouped, int MG, bool kPre, int D, bool kOdd, bool kLoop>
 __global__ __launch_bounds__(kSkinnyWaves * 64) __attribute__((amdgpu_waves_per_eu(kGrouped ? 4 : 2))) void q4_skinny_kernel(
     SkinnyArgs a) {
     static_assert(MG == 1 || (MG == 2 && !kGrouped), "two row groups in dense mode only");
@@ -124,6 +136,7 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) __attribute__((amdgpu_waves_per_
     static_assert(!(kPre && (kGrouped || kGateUp)), "bias and accumulation: dense plain tiles only");
     static_assert(D == 2 || (D == 3 && !kGrouped), "a deeper ring in dense mode only");
     static_assert(!kPre || D == 2, "epilogue operands with one tile in flight only");
+    static_assert(!kLoop || (!kGrouped && D == 2), "a slab loop in dense mode only");
     constexpr int NW = kSkinnyWaves;
     constexpr int KW = kSkinnyPieces;                  // 128-column pieces per wave
     constexpr uint32_t kTileRows = kGateUp ? 8 : 16;  // output features per tile
@@ -131,20 +144,28 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) __attribute__((amdgpu_waves_per_
     constexpr int kStage = 16 * kUnits / (NW * 64);    // X units staged per thread
     __shared__ u32x4 xs[16 * kUnits];                  // X slab: 16 rows x kSlabCols bf16
     __shared__ float red[2][MG][NW][4][64];            // per-wave partial tiles, double buffered
+    __shared__ float sums[kLoop ? kLoopTiles : 1][kLoop ? MG * 256 : 1];  // kLoop: per tile, of the slabs so far
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 4, r16 = lane & 15;
     const uint32_t K = a.k;
-    const uint32_t slab = blockIdx.x % a.ksplit;
-    const uint32_t k0 = slab * (uint32_t)kSlabCols;
+    uint32_t slab = kLoop ? 0u : blockIdx.x % a.ksplit;
+    uint32_t k0 = slab * (uint32_t)kSlabCols;
     // live pieces of the slab (the last one half when K % 128 == 64) and live 8-column X units
-    const uint32_t npieces = min((uint32_t)(NW * KW), (K - k0 + 127) >> 7);
-    const uint32_t kunits = min((uint32_t)(NW * KW * 16), (K - k0) >> 3);
+    uint32_t npieces = min((uint32_t)(NW * KW), (K - k0 + 127) >> 7);
+    uint32_t kunits = min((uint32_t)(NW * KW * 16), (K - k0) >> 3);
+    const uint32_t nslab = kLoop ? (K + kSlabCols - 1) / kSlabCols : 1u;
+    uint32_t tile0 = 0;  // kLoop: the tile (of the current problem) that sums[0] belongs to
     const uint32_t p0 = (uint32_t)wave * KW;                           // this wave's first piece
-    const uint32_t kMask = opq_s(0x000F000Fu);
-    const uint32_t kMagic = opq_v(0x43004300u);  // bf16 128.0 in both halves
+    // B = 128 + q; the slab loop, whose launches had f32 sums of fp16 weights before it, 16 + q: at n = 2048, K =
+    // 11008, m = 27 its error against 64 bits is 1.7e-7 (about
+    // 1.2e-6 with 128 + q, 4.6e-7 on the prefill kernel)
+    constexpr float kOffset = kLoop ? -16.0f : -128.0f;
+    const uint32_t kMask = kLoop ? opq_s(0x00780078u) : opq_s(0x000F000Fu);
+    const uint32_t kMagic = kLoop ? opq_v(0x41804180u) : opq_v(0x43004300u);  // bf16 16.0 or 128.0 in both halves
+    auto frag = [&](uint32_t q) { return kLoop ? q_frag16(q, kMask, kMagic) : q_frag(q, kMask, kMagic); };
 
     // ---- active experts (grouped mode), held in registers: lane l covers experts l + 64 i
     constexpr int kEPer = kGrouped ? (int)(kMaxExperts / 64) : 1;
@@ -461,8 +482,8 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) __attribute__((amdgpu_waves_per_
 #pragma unroll
             for (int h = 0; h < 2; ++h) {  // one group at a time: fewer registers live
                 const float sg = __uint_as_float(h ? (sv & 0xFFFF0000u) : (sv << 16));
-                const float cg = fmaf(-128.0f, sg, __uint_as_float(h ? (bv & 0xFFFF0000u) : (bv << 16)));
-                const bf16x8_t q01 = q_frag(p01[h], kMask, kMagic), q23 = q_frag(p23[h], kMask, kMagic);
+                const float cg = fmaf(kOffset, sg, __uint_as_float(h ? (bv & 0xFFFF0000u) : (bv << 16)));
+                const bf16x8_t q01 = frag(p01[h]), q23 = frag(p23[h]);
 #pragma unroll
                 for (int gi = 0; gi < MG; ++gi) {  // the unpacked words serve every row group
                     bf16x8_t xp[2];
@@ -515,14 +536,28 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) __attribute__((amdgpu_waves_per_
                 __hip_atomic_store(dst + ((kGateUp && ecol >= 8) ? crows : 0u) + f, val, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
             } else {
+                float up = 0.0f;
                 if constexpr (kGateUp) {
-                    float up = 0.0f;
 #pragma unroll
                     for (int w = 0; w < NW; ++w) up += red[par][eg][w][v][L + 8];
-                    val = activation(val, a.act) * up;
                 }
+                bool store = true;
+                if constexpr (kLoop) {  // gate/up: the up sum in the slot of column + 8, whose thread has no output
+                    float *sum = &sums[t - tile0][tid];
+                    if (slab > 0) {
+                        val += sum[0];
+                        if constexpr (kGateUp) up += sum[8];
+                    }
+                    store = slab + 1 == nslab;
+                    if (!store) {
+                        sum[0] = val;
+                        if constexpr (kGateUp) sum[8] = up;
+                    }
+                }
+                if constexpr (kGateUp) val = activation(val, a.act) * up;
                 const size_t o = (size_t)orow * cldo + f;
-                if constexpr (kPre) {
+                if (!store) {
+                } else if constexpr (kPre) {
                     if (cbias) val += __uint_as_float(pre_b[b] << 16);
                     if (a.out_f32) {
                         reinterpret_cast<float *>(cout)[o] = a.accumulate ? __uint_as_float(pre_o[b]) + val : val;
@@ -700,9 +735,11 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) __attribute__((amdgpu_waves_per_
     };
 
     if constexpr (!kGrouped) {  // dense: one X for the whole run
-        const uint32_t rows = min(a.m, 16u * MG);
+        // slab loop: blockIdx.y is the group of 16 MG token rows
+        const uint32_t row0 = kLoop ? 16u * MG * blockIdx.y : 0u;
+        const uint32_t rows = min(a.m - row0, 16u * MG);
         eout = tid < 256 * MG && erow < rows && (!kGateUp || a.partial || ecol < 8);
-        orow = erow;
+        orow = row0 + erow;
         // the problem holding tile t: its fields, by value; returns its first tile
         auto select = [&](uint32_t t) -> uint32_t {
             const int pi = (a.nmore > 1 && t >= a.tile_begin[2]) ? 2 : (a.nmore > 0 && t >= a.tile_begin[1]) ? 1 : 0;
@@ -730,6 +767,43 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) __attribute__((amdgpu_waves_per_
             if (a.nmore > 1 && t < a.tile_begin[2]) return a.tile_begin[2];
             return a.nmore == 0 ? a.tile_begin[1] : a.nmore == 1 ? a.tile_begin[2] : a.tile_begin[3];
         };
+        if constexpr (kLoop) {
+            for (uint32_t first = run_begin; first < run_end; first += kLoopTiles) {
+                const uint32_t last = min(first + kLoopTiles, run_end);
+                for (slab = 0; slab < nslab; ++slab) {
+                    k0 = slab * (uint32_t)kSlabCols;
+                    npieces = min((uint32_t)(NW * KW), (K - k0 + 127) >> 7);
+                    kunits = min((uint32_t)(NW * KW * 16), (K - k0) >> 3);
+                    // X and the tiles as below (every wave has read the last slab's fragments: its tiles ended at
+                    // barriers since); a last group of 16 rows or fewer repeats row row0 with no live rows
+                    uint32_t tb = select(first);
+                    const uint32_t rows0 = min(rows, 16u), rows1 = rows - rows0;
+                    stage_load(raw[0], row0, rows0);
+                    if constexpr (MG == 2) stage_load(raw[MG - 1], rows1 ? row0 + 16 : row0, rows1);
+                    fetch(B0{}, 0, first - tb);
+                    __builtin_amdgcn_sched_barrier(0);
+                    stage_store(raw[0], rows0);
+                    lds_barrier();
+                    load_x_frags(std::integral_constant<int, 0>{});
+                    if constexpr (MG == 2) {
+                        lds_barrier();
+                        stage_store(raw[MG - 1], rows1);
+                        lds_barrier();
+                        load_x_frags(std::integral_constant<int, MG - 1>{});
+                    }
+                    for (uint32_t t = first;;) {
+                        const uint32_t seg_end = min(last, next_begin(t));
+                        tile0 = first - tb;  // sums[t - first]: unsigned wrap past a problem's first tile
+                        run_tiles(0, t - tb, seg_end - tb);
+                        t = seg_end;
+                        if (t >= last) break;
+                        tb = select(t);
+                        fetch(B0{}, 0, t - tb);
+                    }
+                }
+            }
+            return;
+        }
         uint32_t tb = select(run_begin);
         // X loads first (every row group's), then the first tile's words: the conversion waits for
         // X only.  The row groups pass through the one LDS slab in turn (the launcher gives a
@@ -795,8 +869,31 @@ namespace {
 template <bool GU, bool G, int MG, bool P, int D, bool O>
 hipError_t launch_d(SkinnyArgs &a, uint32_t nblk, hipStream_t s) {
     const dim3 grid(nblk * a.ksplit), block(kSkinnyWaves * 64);
-    hipLaunchKernelGGL((q4_skinny_kernel<GU, G, MG, P, D, O>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((q4_skinny_kernel<GU, G, MG, P, D, O, false>), grid, block, 0, s, a);
     return hipGetLastError();
+}
+
+// The slab loop: a block per run of tiles and group of 16 MG token rows, all K slabs inside.
+template <bool GU, int MG>
+hipError_t launch_loop(SkinnyArgs &a, uint32_t items, hipStream_t s) {
+    a.ksplit = 1;
+    const uint32_t groups = (a.m + 16 * MG - 1) / (16 * MG);
+    const uint32_t cap = std::max<uint32_t>(1, (uint32_t)tuning().skinny_max_blocks / groups);
+    const dim3 grid(std::max<uint32_t>(1, std::min(items, cap)), groups), block(kSkinnyWaves * 64);
+    if (a.k % 128 == 0)
+        hipLaunchKernelGGL((q4_skinny_kernel<GU, false, MG, !GU, 2, false, true>), grid, block, 0, s, a);
+    else
+        hipLaunchKernelGGL((q4_skinny_kernel<GU, false, MG, !GU, 2, true, true>), grid, block, 0, s, a);
+    return hipGetLastError();
+}
+
+// Estimated microseconds of a slab-loop launch over `tiles` weight tiles in groups of 16 mg rows: per slab, the
+// staging of X and the block's tiles (measured: n = 2048, K = 11008, 6 slabs: 16 rows 17.4 us, 32 rows 28.1;
+// gate/up [2 x 9536, 3072], 2 slabs of 5 tiles: 17.1 and 22.3).
+float loop_us(uint32_t m, uint32_t tiles, uint32_t k, uint32_t mg) {
+    const uint32_t groups = (m + 16 * mg - 1) / (16 * mg), cap = std::max<uint32_t>(1, 256 / groups);
+    const float per = (float)((tiles + cap - 1) / cap);
+    return (float)skinny_ksplit(k) * (mg == 1 ? 1.6f + 1.3f * per : 2.8f + 1.8f * per);
 }
 
 template <bool GU, bool G, int MG, bool P, bool O>
@@ -839,7 +936,8 @@ hipError_t launch_skinny(SkinnyArgs &a, hipStream_t s) {
     if (grouped && (a.ksplit != 1 || a.k % 128 != 0)) return hipErrorInvalidValue;
     if (grouped && (a.nmore > 0 || a.ln_w || a.bias || a.accumulate)) return hipErrorInvalidValue;
     if (a.nmore < 0 || a.nmore > 2 || (a.nmore > 0 && (gate_up || a.partial))) return hipErrorInvalidValue;
-    if (!grouped && (a.m == 0 || a.m > kSkinnyMaxM)) return hipErrorInvalidValue;
+    const bool loop = !grouped && a.ksplit > 1 && !a.partial;
+    if (!grouped && (a.m == 0 || a.m > (loop ? kSkinnyChunkMaxM : kSkinnyMaxM))) return hipErrorInvalidValue;
     if (a.ln_w && a.ksplit != 1) return hipErrorInvalidValue;  // the norm needs the whole row in the slab
     if (a.tickets && (grouped || a.nmore > 0 || !a.partial || a.ksplit < 2 || a.ksplit > kSkinnyMaxTicketSplit))
         return hipErrorInvalidValue;
@@ -866,6 +964,12 @@ hipError_t launch_skinny(SkinnyArgs &a, hipStream_t s) {
         return gate_up ? launch_t<true, true, 1, false, false>(a, items, s)
                        : launch_t<false, true, 1, false, false>(a, items, s);
     if (gate_up && pre) return hipErrorInvalidValue;  // gate/up launches have neither
+    if (loop) {
+        // 16-row groups on more blocks while there are few tiles, else two groups per unpacked word
+        if (a.m > 16 && loop_us(a.m, items, a.k, 2) < loop_us(a.m, items, a.k, 1))
+            return gate_up ? launch_loop<true, 2>(a, items, s) : launch_loop<false, 2>(a, items, s);
+        return gate_up ? launch_loop<true, 1>(a, items, s) : launch_loop<false, 1>(a, items, s);
+    }
     if (a.m > 16) {  // two row groups per launch
         if (gate_up) return launch_dense<true, 2, false>(a, items, s);
         return pre ? launch_dense<false, 2, true>(a, items, s) : launch_dense<false, 2, false>(a, items, s);
@@ -875,6 +979,11 @@ hipError_t launch_skinny(SkinnyArgs &a, hipStream_t s) {
 }
 
 uint32_t skinny_ksplit(uint32_t k) { return (k + kSlabCols - 1) / kSlabCols; }
+
+float skinny_loop_us(uint32_t m, uint32_t rows, uint32_t k, bool gate_up) {
+    const uint32_t tiles = (rows + (gate_up ? 7 : 15)) / (gate_up ? 8 : 16);
+    return m > 16 ? std::min(loop_us(m, tiles, k, 1), loop_us(m, tiles, k, 2)) : loop_us(m, tiles, k, 1);
+}
 
 bool skinny_grouped_fits(uint32_t k) { return k % 128 == 0 && skinny_ksplit(k) == 1; }  // even group counts only
 
