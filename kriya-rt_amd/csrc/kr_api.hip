@@ -677,6 +677,50 @@ int kr_q4_linear_ws(const kr_q4_matrix *w, const uint16_t *x, uint32_t m, void *
     return hip_status(launch_mfma(args, bm, s), "kr_q4_linear_ws");
 }
 
+// kr_q4_mlp, and its norm's part of kr_rmsnorm_q4_mlp: with `ln_weight`, x is first written as the RMSNorm of bf16 h.
+static int run_mlp(const kr_q4_matrix *gate, const kr_q4_matrix *up, const kr_q4_matrix *down, const uint16_t *x, void *h,
+                   int h_dtype, uint32_t m, int activation, void *workspace, void *stream, uint16_t *xnorm,
+                   const uint16_t *ln_weight, float eps) {
+    hipStream_t s = (hipStream_t)stream;
+    uint16_t *act = mlp_ws_act(workspace);
+    if (mlp_prefill_operands(m) && tuning().prefill_kernel != 1 && tuning().prefill_operands) {
+        // Prefill kernel for both: x converted to its fp16 operand order once (not once per block),
+        // and the gate/up epilogue writes the activation in that form too for the down projection
+        // (the bf16 activation stays the exact operand of the kernel's overflow fallback).
+        const Q4Mat g = to_mat(gate), u = to_mat(up);
+        MfmaArgs gu = mfma_args(x, m, gate->k, KR_DTYPE_BF16, 0);
+        gu.act = activation;
+        gu.p[0] = problem(g, &u, act, nullptr, gate->n);
+        gu.np = 1;
+        MfmaArgs dn = mfma_args(act, m, down->k, h_dtype, 1);
+        dn.p[0] = problem(to_mat(down), nullptr, h, nullptr, down->n);
+        dn.np = 1;
+        if (prefill_supported(gu) && prefill_supported(dn)) {
+            uint16_t *xh = mlp_ws_xh(workspace, m, gate->k, gate->n);
+            uint16_t *acth = mlp_ws_acth(workspace, m, gate->k, gate->n);
+            const bool norm_converts = ln_weight && rmsnorm_one_pass(gate->k);
+            if (ln_weight) {
+                const hipError_t e = launch_rmsnorm((const uint16_t *)h, ln_weight, m, gate->k, eps, xnorm, s,
+                                                    norm_converts ? xh : nullptr);
+                if (int rc = hip_status(e, "kr_rmsnorm_q4_mlp")) return rc;
+            }
+            if (!norm_converts)
+                if (int rc = hip_status(launch_x_to_f16(x, m, gate->k, xh, s), "kr_q4_mlp (x to fp16)")) return rc;
+            gu.xh = xh;
+            gu.out_h = acth;
+            if (int rc = hip_status(launch_prefill(gu, s), "kr_q4_mlp (gate/up)")) return rc;
+            dn.xh = acth;
+            choose_split_k(dn, bm_class(m), mlp_ws_partial(workspace, m, gate->n));
+            return hip_status(launch_prefill(dn, s), "kr_q4_mlp (down)");
+        }
+    }
+    if (ln_weight)
+        if (int rc = hip_status(launch_rmsnorm((const uint16_t *)h, ln_weight, m, gate->k, eps, xnorm, s), "kr_rmsnorm_q4_mlp"))
+            return rc;
+    if (int rc = kr_q4_gate_up_act(gate, up, x, m, act, KR_DTYPE_BF16, activation, stream)) return rc;
+    return mlp_down(gate, down, act, h, h_dtype, m, workspace, stream);
+}
+
 int kr_q4_mlp(const kr_q4_matrix *gate, const kr_q4_matrix *up, const kr_q4_matrix *down, const uint16_t *x,
               void *h, int h_dtype, uint32_t m, int activation, void *workspace, size_t workspace_bytes,
               void *stream) {
@@ -700,34 +744,7 @@ int kr_q4_mlp(const kr_q4_matrix *gate, const kr_q4_matrix *up, const kr_q4_matr
     if (!workspace || workspace_bytes < need)
         return fail(KR_E_WORKSPACE, "workspace of %zu bytes required, %zu given", need, workspace_bytes);
     if (!aligned(workspace, 16)) return fail(KR_E_ALIGN, "workspace must be 16-byte aligned");
-    uint16_t *act = mlp_ws_act(workspace);
-    if (mlp_prefill_operands(m) && tuning().prefill_kernel != 1 && tuning().prefill_operands) {
-        // Prefill kernel for both: x converted to its fp16 operand order once (not once per block),
-        // and the gate/up epilogue writes the activation in that form too for the down projection
-        // (the bf16 activation stays the exact operand of the kernel's overflow fallback).
-        const Q4Mat g = to_mat(gate), u = to_mat(up);
-        hipStream_t s = (hipStream_t)stream;
-        MfmaArgs gu = mfma_args(x, m, gate->k, KR_DTYPE_BF16, 0);
-        gu.act = activation;
-        gu.p[0] = problem(g, &u, act, nullptr, gate->n);
-        gu.np = 1;
-        MfmaArgs dn = mfma_args(act, m, down->k, h_dtype, 1);
-        dn.p[0] = problem(to_mat(down), nullptr, h, nullptr, down->n);
-        dn.np = 1;
-        if (prefill_supported(gu) && prefill_supported(dn)) {
-            uint16_t *xh = mlp_ws_xh(workspace, m, gate->k, gate->n);
-            uint16_t *acth = mlp_ws_acth(workspace, m, gate->k, gate->n);
-            if (int rc = hip_status(launch_x_to_f16(x, m, gate->k, xh, s), "kr_q4_mlp (x to fp16)")) return rc;
-            gu.xh = xh;
-            gu.out_h = acth;
-            if (int rc = hip_status(launch_prefill(gu, s), "kr_q4_mlp (gate/up)")) return rc;
-            dn.xh = acth;
-            choose_split_k(dn, bm_class(m), mlp_ws_partial(workspace, m, gate->n));
-            return hip_status(launch_prefill(dn, s), "kr_q4_mlp (down)");
-        }
-    }
-    if (int rc = kr_q4_gate_up_act(gate, up, x, m, act, KR_DTYPE_BF16, activation, stream)) return rc;
-    return mlp_down(gate, down, act, h, h_dtype, m, workspace, stream);
+    return run_mlp(gate, up, down, x, h, h_dtype, m, activation, workspace, stream, nullptr, nullptr, 0.0f);
 }
 
 int kr_moe_route(const float *logits, uint32_t tokens, uint32_t experts, uint32_t topk, int normalize,
@@ -1245,8 +1262,7 @@ int kr_rmsnorm_q4_mlp(const kr_q4_matrix *gate, const kr_q4_matrix *up, const kr
         return mlp_down(gate, down, act, h, KR_DTYPE_BF16, m, workspace, stream);
     }
     uint16_t *xnorm = (uint16_t *)((char *)workspace + mlp_bytes);
-    if (int rc = hip_status(launch_rmsnorm(h, ln_weight, m, gate->k, eps, xnorm, s), "kr_rmsnorm_q4_mlp")) return rc;
-    return kr_q4_mlp(gate, up, down, xnorm, h, KR_DTYPE_BF16, m, activation, workspace, mlp_bytes, stream);
+    return run_mlp(gate, up, down, xnorm, h, KR_DTYPE_BF16, m, activation, workspace, stream, xnorm, ln_weight, eps);
 }
 
 size_t kr_attention_workspace_bytes(uint32_t batch, uint32_t q_heads, uint32_t head_dim, uint32_t max_ctx) {

@@ -263,8 +263,10 @@ bool skinny_supported(const Q4Mat &w);
 constexpr uint32_t kGlueMaxCtx = 8192;
 constexpr uint32_t kGlueMaxHeadDim = 256;
 hipError_t launch_q4_embedding(const Q4Mat &w, const uint32_t *tokens, uint32_t count, uint16_t *out, hipStream_t s);
+// rows that launch_rmsnorm holds in registers; of those it also writes xh, launch_x_to_f16 of `out` (null: it does not)
+__host__ __device__ constexpr bool rmsnorm_one_pass(uint32_t dim) { return dim % 8 == 0 && dim <= 8 * 4 * 256; }
 hipError_t launch_rmsnorm(const uint16_t *x, const uint16_t *weight, uint32_t rows, uint32_t dim, float eps,
-                          uint16_t *out, hipStream_t s);
+                          uint16_t *out, hipStream_t s, uint16_t *xh = nullptr);
 hipError_t launch_rope_kv_append(uint16_t *q, const uint16_t *k, const uint16_t *v, const float *cos_sin,
                                  const uint32_t *positions, uint32_t batch, uint32_t q_heads, uint32_t kv_heads,
                                  uint32_t D, uint16_t *k_cache, uint16_t *v_cache, uint32_t max_ctx, hipStream_t s);
