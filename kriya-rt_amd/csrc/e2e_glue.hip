@@ -43,10 +43,11 @@ __global__ __launch_bounds__(256) void q4_embedding_kernel(Q4Mat w, const uint32
 // One block per row: y = bf16(x * rsqrt(mean(x^2) + eps) * w).  Rows of
 // dim % 8 == 0 and dim <= 8192 take one pass: each thread holds up to four
 // 8-element pieces of x and w in registers from a single round of loads.
-// xh (those rows only, else null): the output once more as the prefill kernels' fp16 operand, x_to_f16_kernel's
+// kOperand (those rows only): xh is the output once more as the prefill kernels' fp16 operand, x_to_f16_kernel's
 // bits.  Bound by launch and load latency (the bf16 pass alone: 3.4 us for 100 rows of 2048, 9.1 for 3907), so the
 // conversion costs little here; as a launch of its own it took 2.6 and 6.9 us.  MLP 2048 x 11008: m = 100 52.1 -> 51.0,
 // m = 512 100.4 -> 98.0, m = 3907 516 -> 509.
+template <bool kOperand>
 __global__ __launch_bounds__(256) void rmsnorm_kernel(const uint16_t *x, const uint16_t *weight, uint32_t dim,
                                                       float eps, uint16_t *out, uint16_t *xh) {
     __shared__ float red[4];
@@ -105,7 +106,7 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const uint16_t *x, const u
                 }
                 const u32x4 y = {o[0], o[1], o[2], o[3]};
                 *reinterpret_cast<u32x4 *>(yr + 8 * pc) = y;
-                if (xh) *reinterpret_cast<u32x4 *>(xh + (size_t)row * dim + 8 * pc) = x_unit_f16(y);
+                if constexpr (kOperand) *reinterpret_cast<u32x4 *>(xh + (size_t)row * dim + 8 * pc) = x_unit_f16(y);
             }
         }
     } else {
@@ -1184,7 +1185,10 @@ hipError_t launch_q4_embedding(const Q4Mat &w, const uint32_t *tokens, uint32_t 
 hipError_t launch_rmsnorm(const uint16_t *x, const uint16_t *weight, uint32_t rows, uint32_t dim, float eps,
                           uint16_t *out, hipStream_t s, uint16_t *xh) {
     if (xh && !rmsnorm_one_pass(dim)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(rmsnorm_kernel, dim3(rows), dim3(256), 0, s, x, weight, dim, eps, out, xh);
+    if (xh)
+        hipLaunchKernelGGL(rmsnorm_kernel<true>, dim3(rows), dim3(256), 0, s, x, weight, dim, eps, out, xh);
+    else
+        hipLaunchKernelGGL(rmsnorm_kernel<false>, dim3(rows), dim3(256), 0, s, x, weight, dim, eps, out, xh);
     return hipGetLastError();
 }
 
