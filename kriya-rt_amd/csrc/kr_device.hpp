@@ -83,6 +83,27 @@ __device__ __forceinline__ float dot2_bf16(uint32_t a, uint32_t b, float c) {
 __device__ __forceinline__ uint32_t pack_lo(uint32_t a, uint32_t b) { return (a & 0xFFFFu) | (b << 16); }
 __device__ __forceinline__ uint32_t pack_hi(uint32_t a, uint32_t b) { return (a >> 16) | (b & 0xFFFF0000u); }
 
+// w[row] . x over columns c0 .. c1 - 1 (multiples of 8) in plain f32, the weights dequantised one by one: the value
+// of an output whose matrix-core sum is not finite (infinite x, or |x| so large that x times an integer offset or an
+// fp16 operand overflows).  x: bf16, 16-byte aligned.
+__device__ __forceinline__ float q4_exact_dot(const Q4Mat &w, size_t row, const uint16_t *x, uint32_t k, uint32_t c0,
+                                              uint32_t c1) {
+    float sum = 0.0f;
+#pragma unroll 1
+    for (uint32_t c = c0; c < c1; c += 8) {
+        const uint32_t q = w.qw[row * (k >> 3) + (c >> 3)];
+        const float s = bf16_to_f32(w.sc[row * (k >> 6) + (c >> 6)]), b = bf16_to_f32(w.bi[row * (k >> 6) + (c >> 6)]);
+        const u32x4 v = *reinterpret_cast<const u32x4 *>(x + c);
+        const uint32_t X[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float xj = __uint_as_float(j & 1 ? X[j >> 1] & 0xFFFF0000u : X[j >> 1] << 16);
+            sum = fmaf(fmaf((float)((q >> (4 * j)) & 15u), s, b), xj, sum);
+        }
+    }
+    return sum;
+}
+
 // ---- loads that do not keep streamed weights in the caches
 template <typename T>
 __device__ __forceinline__ T ld_stream(const T *p) {

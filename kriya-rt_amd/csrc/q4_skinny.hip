@@ -127,7 +127,8 @@ __device__ __forceinline__ uint32_t xs_index(uint32_t r, uint32_t u) {
 // are not 4-byte aligned when K / 64 is odd).
 // kLoop: K longer than one slab with no room for partials (dense mode): a block takes every slab of its tiles in
 // turn, restaging X per slab, and keeps the sums over the slabs so far in LDS (one float per thread and tile, up
-// to kLoopTiles tiles at a time), added in slab order as the split-K reduction does.
+// to kLoopTiles tiles at a time), added in slab order as the split-K reduction does.  An output that comes out
+// non-finite is computed again in plain f32: the launches it took over had that from the prefill kernel.
 template <bool kGateUp, bool kGrouped, int MG, bool kPre, int D, bool kOdd, bool kLoop>
 __global__ __launch_bounds__(kSkinnyWaves * 64) __attribute__((amdgpu_waves_per_eu(kGrouped ? 4 : 2))) void q4_skinny_kernel(
     SkinnyArgs a) {
@@ -158,6 +159,7 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) __attribute__((amdgpu_waves_per_
     uint32_t kunits = min((uint32_t)(NW * KW * 16), (K - k0) >> 3);
     const uint32_t nslab = kLoop ? (K + kSlabCols - 1) / kSlabCols : 1u;
     uint32_t tile0 = 0;  // kLoop: the tile (of the current problem) that sums[0] belongs to
+    uint32_t redo = 0;   // kLoop: bit j: this thread's output of tile tile0 + j is not finite
     const uint32_t p0 = (uint32_t)wave * KW;                           // this wave's first piece
     // B = 128 + q; the slab loop, whose launches had f32 sums of fp16 weights before it, 16 + q: at n = 2048, K =
     // 11008, m = 27 its error against 64 bits is 1.7e-7 (about
@@ -552,6 +554,9 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) __attribute__((amdgpu_waves_per_
                     if (!store) {
                         sum[0] = val;
                         if constexpr (kGateUp) sum[8] = up;
+                    } else if (!(__builtin_isfinite(val) && __builtin_isfinite(up))) {
+                        store = false;  // exact_outputs() writes it
+                        redo |= 1u << (t - tile0);
                     }
                 }
                 if constexpr (kGateUp) val = activation(val, a.act) * up;
@@ -768,6 +773,30 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) __attribute__((amdgpu_waves_per_
             return a.nmore == 0 ? a.tile_begin[1] : a.nmore == 1 ? a.tile_begin[2] : a.tile_begin[3];
         };
         if constexpr (kLoop) {
+            // This thread's outputs of tiles first .. that came out non-finite: s D and (b - 16 s) S overflow, or
+            // meet as opposite infinities, where the sum itself need not.  After the slabs: n = 2048, K =
+            // 11008, m = 27 takes 20.5 us so, 22.4 with the same code inside finish() (which runs per tile).
+            auto exact_outputs = [&](uint32_t first, uint32_t last) {
+                const uint16_t *xr = a.x + (size_t)orow * a.ldx;
+                for (uint32_t T = first; T < last; ++T) {
+                    const bool mine = (redo >> (T - first)) & 1u;
+                    if (!__any(mine)) continue;
+                    const uint32_t f = (T - select(T)) * kTileRows + (ecol & (kTileRows - 1));
+                    if (!mine) continue;
+                    float val = q4_exact_dot(cw, f, xr, K, 0, K);
+                    if constexpr (kGateUp) val = activation(val, a.act) * q4_exact_dot(cw2, f, xr, K, 0, K);
+                    if (cbias) val += bf16_to_f32(cbias[f]);
+                    const size_t o = (size_t)orow * cldo + f;
+                    if (a.out_f32) {
+                        float *out = reinterpret_cast<float *>(cout) + o;
+                        *out = a.accumulate ? *out + val : val;
+                    } else {
+                        uint16_t *out = reinterpret_cast<uint16_t *>(cout) + o;
+                        *out = (uint16_t)f32_to_bf16(a.accumulate ? val + bf16_to_f32(*out) : val);
+                    }
+                }
+                redo = 0;
+            };
             for (uint32_t first = run_begin; first < run_end; first += kLoopTiles) {
                 const uint32_t last = min(first + kLoopTiles, run_end);
                 for (slab = 0; slab < nslab; ++slab) {
@@ -801,6 +830,7 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) __attribute__((amdgpu_waves_per_
                         fetch(B0{}, 0, t - tb);
                     }
                 }
+                if (__any(redo != 0)) exact_outputs(first, last);
             }
             return;
         }

@@ -66,3 +66,58 @@ def test_qkv(kq, m, k):
     for i in range(3):
         want = O.q4_matmul(O.Q4Planar(*ws[i]), x) + O.bf16_to_f32(bs[i])[None, :]
         assert_rms_close(outs[i].cpu().numpy(), want, rel=2e-5, what=f"problem {i}")
+
+
+def beyond_range(x):
+    """Rows 1 .. 5 of x get an infinity of either sign, a NaN, one column and three columns of 3e37 (31 times that
+    overflows f32, times a weight of about 0.1 it does not)."""
+    big = O.bf16_to_f32(x).copy()
+    big[1, 70], big[2, -1], big[3, 5] = np.inf, -np.inf, np.nan
+    big[4, 2050] = 3e37
+    big[5, [0, 100, 2100]] = 3e37, -3e37, 2e37
+    return O.f32_to_bf16(big)
+
+
+def assert_beyond_range(got, want, rel, what):
+    """Infinities and NaNs where the oracle has them; finite rows at the bar, each against its own RMS."""
+    assert np.array_equal(np.isnan(got), np.isnan(want)), what
+    inf = np.isinf(want)
+    assert np.array_equal(np.isinf(got), inf) and np.array_equal(got[inf], want[inf]), what
+    for i in np.nonzero(np.isfinite(want).all(axis=1))[0]:
+        assert_rms_close(got[i], want[i], rel=rel, what=f"{what} row {i}")
+
+
+@pytest.mark.parametrize("m,n,k", [(27, 300, 4160), (63, 33, 2176), (8, 50, 16448)])
+def test_linear_beyond_range(kq, m, n, k):
+    """s D + (b - 16 s) S overflows, or adds opposite infinities, where the product itself does not."""
+    case(f"slab loop linear, infinite and near-maximal x m={m} n={n} k={k}")
+    s = synth()
+    wq, x = s.q4_weight(n, k, 7300 + m), beyond_range(s.bf16_normal((m, k), 7301 + m))
+    want = O.q4_matmul(O.Q4Planar(*wq), x)
+    assert np.isinf(want[1:3]).any() and np.isfinite(want[4:6]).all()
+    got = kq.q4_linear(q4_dev(kq, wq), dev_bf16(x), out_dtype=kq.DTYPE_F32).cpu().numpy()
+    assert_beyond_range(got, want, 2e-5, "f32")
+
+
+@pytest.mark.parametrize("m,n,k,act", [(16, 35, 2112, 2), (27, 300, 4096, 0)])
+def test_gate_up_beyond_range(kq, m, n, k, act):
+    case(f"slab loop gate_up, infinite and near-maximal x m={m} n={n} k={k} activation={act}")
+    s = synth()
+    g, u, x = s.q4_weight(n, k, 7400), s.q4_weight(n, k, 7401), beyond_range(s.bf16_normal((m, k), 7402))
+    x[4:6] = s.bf16_normal((2, k), 7403)  # gate times up of such rows leaves f32's range
+    want = O.q4_gate_up_act(O.Q4Planar(*g), O.Q4Planar(*u), x, act)
+    got = kq.gate_up_act(q4_dev(kq, g), q4_dev(kq, u), dev_bf16(x), activation=act).cpu().numpy()
+    assert_beyond_range(got, want, 1e-2, "f32")
+
+
+def test_qkv_beyond_range(kq):
+    case("slab loop qkv, infinite and near-maximal x m=16 k=2112")
+    s = synth()
+    m, k, ns = 16, 2112, (500, 40, 300)
+    x = beyond_range(s.bf16_normal((m, k), 7500))
+    ws = [s.q4_weight(n, k, 7501 + i) for i, n in enumerate(ns)]
+    bs = [s.bf16_normal((1, n), 7510 + i)[0] for i, n in enumerate(ns)]
+    outs = kq.qkv(*[q4_dev(kq, w) for w in ws], dev_bf16(x), *[dev_bf16(b) for b in bs], out_dtype=kq.DTYPE_F32)
+    for i in range(3):
+        want = O.q4_matmul(O.Q4Planar(*ws[i]), x) + O.bf16_to_f32(bs[i])[None, :]
+        assert_beyond_range(outs[i].cpu().numpy(), want, 2e-5, f"problem {i}")
