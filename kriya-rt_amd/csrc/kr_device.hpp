@@ -85,7 +85,8 @@ __device__ __forceinline__ uint32_t pack_hi(uint32_t a, uint32_t b) { return (a 
 
 // w[row] . x over columns c0 .. c1 - 1 (multiples of 8) in plain f32, the weights dequantised one by one: the value
 // of an output whose matrix-core sum is not finite (infinite x, or |x| so large that x times an integer offset or an
-// fp16 operand overflows).  x: bf16, 16-byte aligned.
+// fp16 operand overflows).  x: bf16, 16-byte aligned; kPairs: every 8 columns in the order e0 e4 e1 e5 e2 e6 e3 e7.
+template <bool kPairs = false>
 __device__ __forceinline__ float q4_exact_dot(const Q4Mat &w, size_t row, const uint16_t *x, uint32_t k, uint32_t c0,
                                               uint32_t c1) {
     float sum = 0.0f;
@@ -97,7 +98,8 @@ __device__ __forceinline__ float q4_exact_dot(const Q4Mat &w, size_t row, const 
         const uint32_t X[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            const float xj = __uint_as_float(j & 1 ? X[j >> 1] & 0xFFFF0000u : X[j >> 1] << 16);
+            const int word = kPairs ? j & 3 : j >> 1, half = kPairs ? j >> 2 : j & 1;
+            const float xj = __uint_as_float(half ? X[word] & 0xFFFF0000u : X[word] << 16);
             sum = fmaf(fmaf((float)((q >> (4 * j)) & 15u), s, b), xj, sum);
         }
     }

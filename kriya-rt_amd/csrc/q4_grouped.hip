@@ -284,6 +284,20 @@ __global__ __launch_bounds__(256, OCC) void q4_grouped_kernel(GroupedArgs a) {
 
     // ---- epilogue, 32 tokens at a time through LDS (a lane holds column c, rows 8 q + 4 h + v of a fragment)
     float *tile = reinterpret_cast<float *>(lds);
+    // Non-finite sums (an infinite x, or |x| beyond about 2e36, whose product with 128 + q overflows) are computed
+    // again in plain f32: the three parts of an infinite S cannot meet b and -128 s.
+    auto finite8 = [](const float *g, int second) {  // 8 sums, and the 8 at + second; 0 times a non-finite one is NaN
+        float z = 0.0f;
+#pragma unroll
+        for (int v = 0; v < 8; ++v) z = fmaf(g[second + v], 0.0f, fmaf(g[v], 0.0f, z));
+        return z == z;
+    };
+    auto exact8 = [&](const Q4Mat &Wm, float *g, uint32_t p, uint32_t n) {
+        const uint16_t *xr = reinterpret_cast<const uint16_t *>(a.xp) + (size_t)(a.x_div ? a.sorted[p] / a.x_div : p) * K;
+#pragma unroll 1
+        for (int v = 0; v < 8; ++v)
+            if (!__builtin_isfinite(g[v])) g[v] = q4_exact_dot<true>(Wm, er + n + v, xr, K, 0, K);
+    };
     static_for<MF>([&](auto Mi) {
         constexpr int m = Mi;
         if ((uint32_t)m >= na) return;
@@ -294,15 +308,20 @@ __global__ __launch_bounds__(256, OCC) void q4_grouped_kernel(GroupedArgs a) {
         __syncthreads();
         if constexpr (kGateUp) {
             const uint32_t r = (uint32_t)tid >> 3, cu = (uint32_t)tid & 7;
-            const float *g = tile + r * T::kPitch + cu * 8;
+            float *g = tile + r * T::kPitch + cu * 8;
+            const uint32_t n = nt * 64 + cu * 8, p = p0 + 32 * m + r;
+            const bool live = 32 * m + r < rows && n < a.rows;
+            if (live && !finite8(g, 64)) {
+                exact8(a.w, g, p, n);
+                exact8(a.w2, g + 64, p, n);
+            }
             float t[8];
 #pragma unroll
             for (int v = 0; v < 8; ++v) t[v] = activation(g[v], a.act) * g[64 + v];
             u32x4 o = {f32_to_bf16(t[0]) | (f32_to_bf16(t[1]) << 16), f32_to_bf16(t[2]) | (f32_to_bf16(t[3]) << 16),
                        f32_to_bf16(t[4]) | (f32_to_bf16(t[5]) << 16), f32_to_bf16(t[6]) | (f32_to_bf16(t[7]) << 16)};
             const float s = group_sum(o);
-            const uint32_t n = nt * 64 + cu * 8, p = p0 + 32 * m + r;
-            if (32 * m + r < rows && n < a.rows) {
+            if (live) {
                 *reinterpret_cast<u32x4 *>(a.out_h + (size_t)p * a.rows + n) = pair_order(o);
                 if (cu == 0) a.out_su[(size_t)p * (a.rows >> 6) + nt] = sum_unit(s);
             }
@@ -312,7 +331,9 @@ __global__ __launch_bounds__(256, OCC) void q4_grouped_kernel(GroupedArgs a) {
                 const uint32_t r = (uint32_t)(tid + 256 * it) >> 4, cu = (uint32_t)tid & 15;
                 const uint32_t n = nt * 128 + cu * 8;
                 if (32 * m + r < rows && n < a.rows) {
-                    const f32x4 *src = reinterpret_cast<const f32x4 *>(tile + r * T::kPitch + cu * 8);
+                    float *g = tile + r * T::kPitch + cu * 8;
+                    if (!finite8(g, 0)) exact8(a.w, g, p0 + 32 * m + r, n);
+                    const f32x4 *src = reinterpret_cast<const f32x4 *>(g);
                     f32x4 *dst = reinterpret_cast<f32x4 *>(a.out_d + (size_t)a.sorted[p0 + 32 * m + r] * a.rows + n);
                     dst[0] = src[0];
                     dst[1] = src[1];

@@ -116,3 +116,29 @@ def test_scan_scatter_many(kq, n, E):
     assert np.array_equal(counts.cpu().numpy(), np.bincount(ids, minlength=E + 1)[:E])
     assert int(offsets[-1]) == want.size
     assert np.array_equal(scatter.cpu().numpy()[: want.size], want)
+
+
+def test_beyond_range(kq):
+    """Weights of one sign, b >= 128 s: an infinite x gives infinite outputs, no NaN from the split S; a row whose
+    activations times 128 + q leave f32's range stays finite."""
+    case("grouped experts, infinite and near-maximal activations")
+    E, hidden, inter, counts = 2, 256, 128, (50, 40)
+    ids = bucketed(counts, E)
+    (g, u, d), x, w, r = setup(kq, ids, E, hidden, inter, 6400)
+
+    def positive(m):  # the same nibbles, scale 2^-10, bias 0.25
+        return m[0], np.full_like(m[1], 0x3A80), np.full_like(m[2], 0x3E80)
+
+    g, u, d = positive(g), positive(u), positive(d)
+    xs = np.abs(O.bf16_to_f32(x)) * 1e-2
+    xs[3, 200], xs[7, 0], xs[9, 100] = np.inf, np.inf, np.nan
+    xs[20] *= 1e18  # activations of about 2e35: 64 of them times 128 + q leave f32, times 0.25 they do not
+    x = O.f32_to_bf16(xs)
+    want = O.moe_experts(O.Q4Planar(*g), O.Q4Planar(*u), O.Q4Planar(*d), E, x, ids, w, 0)
+    assert np.isposinf(want[[3, 7]]).all() and np.isnan(want[9]).all() and np.isfinite(want[20]).all() and want[20].min() > 1e36
+    y = kq.moe_experts(q4_dev(kq, g), q4_dev(kq, u), q4_dev(kq, d), E, dev_bf16(x), r).cpu().numpy()
+    assert np.array_equal(np.isnan(y), np.isnan(want))
+    assert np.array_equal(np.isposinf(y), np.isposinf(want))
+    for t in range(len(ids)):
+        if np.isfinite(want[t]).all():
+            assert_rms_close(y[t] / rms(want[t]), want[t] / rms(want[t]), what=f"token {t}")
