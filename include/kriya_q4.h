@@ -23,7 +23,7 @@
  *     kernels) every bf16 x is multiplied exactly (bf16 products, f32 sums).
  *     For m >= 64 (the prefill kernel) x is staged in fp16, as the reference's
  *     M >= 64 kernels stage half (q4_gemm_and_moe.metal:2722-2724): exact for
- *     |x| in [2^-14, 65504]; a tile whose sums overflow fp16 is recomputed in
+ *     |x| in [2^-14, 65504]; outputs whose sums overflow fp16 are recomputed in
  *     f32 (exact), and values below 2^-14 keep fp16's subnormal precision
  *     (absolute error <= 2^-25 per element).  Weights are rounded once to fp16
  *     there (w = fma(q, s, b)); elsewhere they are exact.

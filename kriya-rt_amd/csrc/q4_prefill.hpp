@@ -1,5 +1,5 @@
 // q4_prefill.hpp — device helpers shared by the prefill kernels (q4_prefill.hip, q4_prefill_wide.hip):
-// buffer resources, direct-to-LDS loads, fp16 operands, the epilogue's stores and the exact f32 tile.
+// buffer resources, direct-to-LDS loads, fp16 operands and the epilogue's stores.
 #pragma once
 
 #include "kr_internal.hpp"
@@ -65,61 +65,6 @@ __device__ __forceinline__ u32x4 x_unit_f16(u32x4 d) {
                  __builtin_bit_cast(uint32_t, o2), __builtin_bit_cast(uint32_t, o3)};
 }
 
-
-// The tile [m0, m0 + rows) x [n0, n0 + cols) of columns [c0, c1) in plain f32 (dequantised weights times
-// bf16 x, exact products of the inputs' values): the path of a block whose fp16 operands overflowed.
-// Rows beyond M and columns beyond N are skipped; it writes the outputs itself.
-template <int EPI, int NW>
-__device__ __forceinline__ void prefill_exact_tile(const MfmaArgs &args, const MfmaProblem &P, uint32_t ks, uint32_t m0,
-                                                uint32_t n0, uint32_t rows, uint32_t cols, uint32_t c0, uint32_t c1,
-                                                uint32_t tid, uint32_t threads) {
-    const uint32_t N = P.w.n, M = args.m, K = args.k, G = K >> 6;
-    for (uint32_t o = tid; o < rows * cols; o += threads) {
-        const uint32_t m = m0 + o / cols, n = n0 + o % cols;
-        if (m >= M || n >= N) continue;
-        float gsum = 0.0f, usum = 0.0f;
-        const uint16_t *xr = args.x + (size_t)m * args.ldx;
-        for (uint32_t c = c0; c < c1; c += 8) {
-            const uint32_t wq = P.w.qw[(size_t)n * (K >> 3) + (c >> 3)];
-            const float sc = bf16_to_f32(P.w.sc[(size_t)n * G + (c >> 6)]), bi = bf16_to_f32(P.w.bi[(size_t)n * G + (c >> 6)]);
-            uint32_t uq = 0;
-            float usc = 0.0f, ubi = 0.0f;
-            if (NW == 2) {
-                uq = P.w2.qw[(size_t)n * (K >> 3) + (c >> 3)];
-                usc = bf16_to_f32(P.w2.sc[(size_t)n * G + (c >> 6)]);
-                ubi = bf16_to_f32(P.w2.bi[(size_t)n * G + (c >> 6)]);
-            }
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float x = bf16_to_f32(xr[c + j]);
-                gsum = fmaf(fmaf((float)((wq >> (4 * j)) & 15u), sc, bi), x, gsum);
-                if (NW == 2) usum = fmaf(fmaf((float)((uq >> (4 * j)) & 15u), usc, ubi), x, usum);
-            }
-        }
-        if (EPI == kMfmaPartial) {
-            float *dst = args.partial + ((size_t)ks * M + m) * (size_t)(NW * N) + n;
-            dst[0] = gsum;
-            if (NW == 2) dst[N] = usum;
-            continue;
-        }
-        float val = gsum;
-        if (NW == 2) val = activation(val, args.act) * usum;
-        if (EPI == kMfmaDirect && P.bias) val += bf16_to_f32(P.bias[n]);
-        const size_t oo = (size_t)m * P.ldo + n;
-        if (args.out_f32) {
-            float *out = reinterpret_cast<float *>(P.out);
-            out[oo] = args.accumulate ? out[oo] + val : val;
-        } else {
-            uint16_t *out = reinterpret_cast<uint16_t *>(P.out);
-            const uint32_t b = f32_to_bf16(args.accumulate ? val + bf16_to_f32(out[oo]) : val);
-            out[oo] = (uint16_t)b;
-            if (NW == 2 && args.out_h) {  // column n of its 8-column unit goes to 2 (n % 4) + (n % 8) / 4
-                const _Float16 hv = (_Float16)bf16_to_f32(b);
-                args.out_h[oo - n + (n & ~7u) + 2 * (n & 3u) + ((n & 7u) >> 2)] = __builtin_bit_cast(uint16_t, hv);
-            }
-        }
-    }
-}
 
 // 16-byte epilogue accesses: the launch's outputs (or partials) and bias allow them.
 template <int EPI>

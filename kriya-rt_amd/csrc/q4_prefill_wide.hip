@@ -36,13 +36,43 @@ namespace kr {
 
 namespace {
 
+// Those of src[0 .. 7] (outputs n .. n + 7 of x) that are not finite, again in plain f32 over columns c0 .. c1 - 1.  All
+// eight at a time: their loads overlap.  Only these outputs: one row of 1e5 in 512, [12288, 4096], takes 1.15 ms (whole
+// tiles: 26.7, 11.8 with the 64 x 64 tiles of q4_prefill.hip).
+__device__ __forceinline__ void exact8(const Q4Mat &w, uint32_t n, const uint16_t *x, uint32_t K, uint32_t c0, uint32_t c1,
+                                       float *src) {
+    bool any = false;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) any |= !__builtin_isfinite(src[e]);
+    if (!any) return;
+    float sum[8] = {};
+#pragma unroll 1
+    for (uint32_t c = c0; c < c1; c += 8) {
+        const u32x4 v = *reinterpret_cast<const u32x4 *>(x + c);
+        const uint32_t X[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const size_t row = min(n + e, w.n - 1);
+            const uint32_t q = w.qw[row * (K >> 3) + (c >> 3)];
+            const float s = bf16_to_f32(w.sc[row * (K >> 6) + (c >> 6)]), b = bf16_to_f32(w.bi[row * (K >> 6) + (c >> 6)]);
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                sum[e] = fmaf(fmaf((float)((q >> (4 * j)) & 15u), s, b),
+                              __uint_as_float(j & 1 ? X[j >> 1] & 0xFFFF0000u : X[j >> 1] << 16), sum[e]);
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+        if (!__builtin_isfinite(src[e])) src[e] = sum[e];
+}
+
 // MF x 32 token rows by 4 waves x NF x 32 weight rows per block.
 template <int MF, int NF, int NW>
 struct WideTile {
     static constexpr int kBM = MF * 32;
     static constexpr int kCols = 4 * NF * 32 / NW;   // output columns per block
     static constexpr int kBuf = kBM * 256;           // one 128-column X slice in fp16
-    static constexpr int kTile = 256 + 4 * 32 * (NF * 32 + 4) * 4;  // the epilogue's LDS tiles, past the flags
+    static constexpr int kTile = 4 * 32 * (NF * 32 + 4) * 4;  // the epilogue's LDS tiles
     static constexpr int kLds = 2 * kBuf > kTile ? 2 * kBuf : kTile;
 };
 
@@ -302,7 +332,8 @@ __global__ __launch_bounds__(256, OCC) void q4_prefill_wide_kernel(MfmaArgs args
         if (i < nsteps) step(std::integral_constant<int, 0>{}, i);
     }
 
-    // 0 * acc is NaN where acc is not finite
+    // A non-finite sum (an operand beyond fp16, or an infinite input: it never turns finite again) is computed again
+    // below, in plain f32; 0 * acc is NaN where acc is not finite.
     float z[4] = {0, 0, 0, 0};
 #pragma unroll
     for (int a = 0; a < MF; ++a)
@@ -311,21 +342,10 @@ __global__ __launch_bounds__(256, OCC) void q4_prefill_wide_kernel(MfmaArgs args
 #pragma unroll
             for (int v = 0; v < 16; ++v) z[v & 3] = fmaf(acc[a][f][v], 0.0f, z[v & 3]);
     const float zs = (z[0] + z[1]) + (z[2] + z[3]);
-    bool bad;
-    {   // every wave's direct-to-LDS loads have landed before the flags are written over the X buffers
-        int8_t *flags = reinterpret_cast<int8_t *>(lds);
-        const bool any_wave = __ballot(zs != zs) != 0ull;
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        if (lane == 0) flags[wave] = any_wave ? 1 : 0;
-        __syncthreads();
-        bad = (flags[0] | flags[1] | flags[2] | flags[3]) != 0;
-    }
-    if (bad) {
-        prefill_exact_tile<EPI, NW>(args, P, ks, m0, nt * T::kCols, T::kBM, T::kCols, g_begin * 128, min(g_end * 128, K), tid,
-                                    256);
-        return;
-    }
+    const bool bad = __ballot(zs != zs) != 0ull;  // in this wave
+    // every wave's direct-to-LDS loads have landed before a tile is written over the X buffers
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
     // A lane holds, of token row c, the weight rows 8 q + 4 h + 0 .. 3 of each fragment: four consecutive
     // columns.  Each wave passes 32 rows at a time through its own LDS region (no block barriers) and
     // stores eight consecutive columns per lane.
@@ -333,7 +353,7 @@ __global__ __launch_bounds__(256, OCC) void q4_prefill_wide_kernel(MfmaArgs args
     constexpr int kWCols = kPair ? 32 : NF * 32;           // columns a wave writes
     constexpr int kPitch = NF * 32 + 4;
     static_assert(NW == 1 || NF == 2, "gate/up waves hold whole pairs");
-    float *tile = reinterpret_cast<float *>(lds + 256) + wave * 32 * kPitch;
+    float *tile = reinterpret_cast<float *>(lds) + wave * 32 * kPitch;
     const bool vec = prefill_vec_out<EPI>(args, P);
     const uint32_t n0 = nt * T::kCols + wave * kWCols;
 #pragma unroll
@@ -347,6 +367,21 @@ __global__ __launch_bounds__(256, OCC) void q4_prefill_wide_kernel(MfmaArgs args
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
         constexpr int kUnits = kWCols / 8;
+        if (bad) {
+            const uint32_t c0 = g_begin * 128, c1 = min(g_end * 128, K);
+#pragma unroll 1
+            for (int it = 0; it < kUnits / 2; ++it) {
+                const uint32_t r = (it * 64 + lane) / kUnits, cu = lane % kUnits;
+                const uint32_t m = m0 + p * 32 + r, n = n0 + cu * 8;
+                if (m >= M || n >= N) continue;
+                const uint16_t *xr = args.x + (size_t)m * args.ldx;
+                float *src = tile + r * kPitch + cu * 8;
+                exact8(P.w, n, xr, K, c0, c1, src);
+                if constexpr (kPair) exact8(P.w2, n, xr, K, c0, c1, src + 32);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
 #pragma unroll 2
         for (int it = 0; it < kUnits / 2; ++it) {
             const uint32_t r = (it * 64 + lane) / kUnits, cu = lane % kUnits;

@@ -108,3 +108,26 @@ def test_fp16_overflow_rows_exact(kq):
     got = kq.q4_linear(q4_dev(kq, wq), dev_bf16(x), out_dtype=kq.DTYPE_F32).cpu().numpy()
     for i in range(m):
         assert_rms_close(got[i], want[i], what=f"row {i}")
+
+
+@pytest.mark.parametrize("m,n,k", [(129, 24573, 128), (65, 24568, 640), (64, 65521, 128)])
+def test_overflow_leaves_other_outputs(kq, m, n, k):
+    """Only outputs that are not finite are computed again: rows beside one beyond fp16's range keep their bits, and
+    infinities and NaNs come out as the oracle has them."""
+    case(f"wide prefill, rows beside an overflowing one m={m} n={n} k={k}")
+    s = synth()
+    wq, x = s.q4_weight(n, k, 5600 + m), s.bf16_normal((m, k), 5601 + m)
+    w = q4_dev(kq, wq)
+    plain = kq.q4_linear(w, dev_bf16(x), out_dtype=kq.DTYPE_F32).cpu().numpy()
+    big = O.bf16_to_f32(x).copy()
+    big[7, 3], big[40, 100], big[m - 1, k - 1], big[12, 0] = 1e5, np.inf, -np.inf, np.nan
+    rows = [7, 40, m - 1, 12]
+    xb = O.f32_to_bf16(big)
+    got = kq.q4_linear(w, dev_bf16(xb), out_dtype=kq.DTYPE_F32).cpu().numpy()
+    others = np.setdiff1d(np.arange(m), rows)
+    assert np.array_equal(got[others].view(np.uint32), plain[others].view(np.uint32))
+    want = O.q4_matmul(O.Q4Planar(*wq), xb[rows])
+    assert_rms_close(got[7], want[0], what="row 7")
+    assert np.array_equal(np.isnan(got[rows]), np.isnan(want)) and np.isnan(want[3]).all()
+    inf = np.isinf(want)
+    assert inf.any() and np.array_equal(np.isinf(got[rows]), inf) and np.array_equal(got[rows][inf], want[inf])
