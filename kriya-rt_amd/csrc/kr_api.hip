@@ -13,6 +13,7 @@
 #include "kriya_glue.h"
 #include "kriya_q4.h"
 #include "kr_internal.hpp"
+#include "launch_rules.hpp"
 
 namespace kr {
 
@@ -219,29 +220,27 @@ size_t partial_bytes(uint32_t m, uint32_t n, uint32_t k, int nw) {
     return round_up((size_t)ks * m * nw * n * 4, 256);
 }
 
-// Split K over the blocks when the tile grid alone would leave CUs idle.
-void choose_split_k(MfmaArgs &a, int bm, float *partial) {
-    const uint32_t groups = a.k / 64;
+// The K split (into `partial`, room for kMaxSplitK) and, on the prefill kernels, the launch shape.  mlp: kr_q4_mlp's
+// down projection, whose x may come converted.
+void choose_split_k(MfmaArgs &a, int bm, float *partial, bool mlp) {
+    const uint32_t groups = a.k / 64, n = a.p[0].w.n, cus = (uint32_t)device_cus();
     const bool prefill = bm > 16 && tuning().prefill_kernel != 1 && prefill_supported(a);
-    if (const uint32_t wide = prefill ? prefill_wide_split(a, kMaxSplitK) : 0) {
-        if (wide > 1) {
-            a.ksplit = wide;
-            a.groups_per_split = ((groups + wide - 1) / wide + 1) & ~1u;
-            a.partial = partial;
-        }
-        return;
-    }
-    const uint32_t rows = prefill ? prefill_block_m(a.p[0].w2.qw != nullptr) : (uint32_t)bm_rows(bm);
-    const uint32_t cols = prefill ? prefill_block_rows(a.p[0].w2.qw != nullptr) : (uint32_t)bn_of(bm, false);
-    const uint32_t tiles = ((a.m + rows - 1) / rows) * ((a.p[0].w.n + cols - 1) / cols);
-    // the prefill kernel's split tiles: about one block per CU (fewer partials to reduce); the
-    // tiled kernel: two
-    const uint32_t target = (prefill ? 1u : 2u) * (uint32_t)device_cus();
     uint32_t split = 1;
-    while (split < kMaxSplitK && tiles * split < target && groups / (split * 2) >= 8) split *= 2;
+    if (prefill && tuning().prefill_kernel == 0 && a.k % 128 == 0) {
+        const PrefillChoice c = prefill_choice(a.m, &n, 1, a.k, kMaxSplitK, mlp, cus);
+        a.prefill_shape = c.shape;
+        split = c.ksplit;
+    } else if (prefill) {
+        a.prefill_shape = kPrefillNarrow;
+        split = narrow_split(a.m, n, a.k, kMaxSplitK, cus);
+    } else {  // the tiled kernel: two blocks per CU
+        const uint32_t rows = (uint32_t)bm_rows(bm), cols = (uint32_t)bn_of(bm, false);
+        const uint32_t tiles = ((a.m + rows - 1) / rows) * ((n + cols - 1) / cols);
+        while (split < kMaxSplitK && tiles * split < 2 * cus && groups / (split * 2) >= 8) split *= 2;
+    }
     if (split > 1) {
         a.ksplit = split;
-        a.groups_per_split = ((groups + split - 1) / split + 1) & ~1u;  // even: the prefill kernel's steps take two groups
+        a.groups_per_split = groups_per_split(a.k, split);
         a.partial = partial;
     }
 }
@@ -635,7 +634,7 @@ static int mlp_down(const kr_q4_matrix *gate, const kr_q4_matrix *down, const ui
     args.p[0] = problem(to_mat(down), nullptr, h, nullptr, down->n);
     args.np = 1;
     const int bm = bm_class(m);
-    choose_split_k(args, bm, partial);
+    choose_split_k(args, bm, partial, true);
     return hip_status(launch_mfma(args, bm, (hipStream_t)stream), "kr_q4_mlp (down)");
 }
 
@@ -673,7 +672,7 @@ int kr_q4_linear_ws(const kr_q4_matrix *w, const uint16_t *x, uint32_t m, void *
     args.p[0] = problem(a, nullptr, y, nullptr, w->n);
     args.np = 1;
     const int bm = bm_class(m);
-    choose_split_k(args, bm, partial);
+    choose_split_k(args, bm, partial, false);
     return hip_status(launch_mfma(args, bm, s), "kr_q4_linear_ws");
 }
 
@@ -710,7 +709,7 @@ static int run_mlp(const kr_q4_matrix *gate, const kr_q4_matrix *up, const kr_q4
             gu.out_h = acth;
             if (int rc = hip_status(launch_prefill(gu, s), "kr_q4_mlp (gate/up)")) return rc;
             dn.xh = acth;
-            choose_split_k(dn, bm_class(m), mlp_ws_partial(workspace, m, gate->n));
+            choose_split_k(dn, bm_class(m), mlp_ws_partial(workspace, m, gate->n), true);
             return hip_status(launch_prefill(dn, s), "kr_q4_mlp (down)");
         }
     }

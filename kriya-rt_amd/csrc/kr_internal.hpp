@@ -108,6 +108,8 @@ struct MfmaArgs {
     // `xcd_tiles` consecutive tiles (see q4_prefill_kernel; the wide kernel uses it as a flag); 0 the
     // default tile grouping
     uint32_t xcd_tiles;
+    // prefill: the launch shape (PrefillShape, launch_rules.hpp); 0: launch_prefill chooses
+    int prefill_shape;
 };
 
 // bm: the M tile class (16, 64 or 128) chosen by the caller from m.
@@ -115,18 +117,13 @@ hipError_t launch_mfma(MfmaArgs &a, int bm, hipStream_t s);
 // Prefill kernel (q4_prefill.hip): m > 16, k % 64 == 0, operands < 4 GiB.
 bool prefill_supported(const MfmaArgs &a);
 hipError_t launch_prefill(MfmaArgs &a, hipStream_t s);
-// The wide-tile prefill kernel (q4_prefill_wide.hip): the shape it takes for a launch (0: it does not), and
-// the number of K splits (a power of two up to max_split; 0: not enough tiles) it wants for a plain
-// projection given room for partials.  launch_prefill picks it by itself.
+// The PrefillShape (launch_rules.hpp) an unsplit launch takes, and the launch of a wide one (q4_prefill_wide.hip).
 int prefill_wide_shape(const MfmaArgs &a);
-uint32_t prefill_wide_split(const MfmaArgs &a, uint32_t max_split);
 hipError_t launch_prefill_wide(MfmaArgs &a, int shape, hipStream_t s);
 // xh[m, k] = fp16 of bf16 x[m, k] (RNE; beyond 65504 -> inf), each 8 columns in the order
 // e0 e4 e1 e5 e2 e6 e3 e7 of the prefill kernel's operands.  k % 8 == 0, 16-byte aligned rows.
 hipError_t launch_x_to_f16(const uint16_t *x, uint32_t m, uint32_t k, uint16_t *xh, hipStream_t s);
 int device_cus();                               // compute units of the current device
-uint32_t prefill_block_m(bool gate_up);         // token rows per block
-uint32_t prefill_block_rows(bool gate_up);      // weight rows (per matrix) per block
 // Fixed-order sum of split-K partials [ksplit, m, nw * N] + the epilogue of p[0].
 hipError_t launch_splitk_reduce(const MfmaArgs &a, int nw, hipStream_t s);
 

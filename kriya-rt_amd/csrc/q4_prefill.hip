@@ -57,8 +57,8 @@
 #include <type_traits>
 
 #include "kr_internal.hpp"
+#include "launch_rules.hpp"
 #include "q4_prefill.hpp"
-
 
 namespace kr {
 
@@ -711,20 +711,14 @@ static hipError_t launch_prefill_shape(MfmaArgs &a, hipStream_t s) {
 // 128-column steps (64-column steps where k / 64 is odd):
 //   gate/up: 128 token rows x (4 waves x 16 gate + 16 up rows), one step of
 //            look-ahead, 2 waves per SIMD (the 32 KB X slices fill the LDS);
-//   plain:    64 token rows x (4 waves x 16 rows), one step of look-ahead, 4
-//             waves per SIMD: the N = 2048 projections are short of blocks with
-//             larger tiles (96 x 128: down 145 us, o 33 us; 64 x 64: 72 / 17.6 us);
+//   plain:   64 token rows x (4 waves x 16 rows): the N = 2048 projections are
+//            short of blocks with larger tiles (96 x 128: down 145 us, o 33 us;
+//            64 x 64: 72 / 17.6 us).  128-column steps: two groups of waves per
+//            tile split them (qkv 20.2 -> 19.0 us; four groups: 21.8 us);
 //   split K: 128 token rows x (4 waves x 32 rows), one step of look-ahead, when
-//             the MLP's workspace lets the down projection split K over blocks
-//             (K split to about one block per CU: cfg2 down 4 ways, 37.0 us + 5.3 us
-//             of reduction, against 96-row tiles split 8 ways, 38.9 + 7.2 us).
-using GateUpShape = PrefillTile<8, 2, 4, 2>;
-using PlainShape = PrefillTile<4, 1, 4, 1>;
-using SplitShape = PrefillTile<8, 2, 4, 1>;  // plain projections whose K is split over blocks
-
-uint32_t prefill_block_m(bool gate_up) { return gate_up ? GateUpShape::kBM : SplitShape::kBM; }
-uint32_t prefill_block_rows(bool gate_up) { return gate_up ? GateUpShape::kBN : SplitShape::kBN; }
-
+//            a workspace lets the projection split K over blocks (to about one
+//            block per CU: cfg2 down 4 ways, 37.0 us + 5.3 us of reduction,
+//            against 96-row tiles split 8 ways, 38.9 + 7.2 us).
 bool prefill_supported(const MfmaArgs &a) {
     // 32-bit buffer offsets: every operand must span < 4 GiB
     const uint64_t xbytes = (uint64_t)a.m * a.ldx * 2;
@@ -737,7 +731,8 @@ bool prefill_supported(const MfmaArgs &a) {
 }
 
 hipError_t launch_prefill(MfmaArgs &a, hipStream_t s) {
-    if (const int shape = prefill_wide_shape(a)) return launch_prefill_wide(a, shape, s);
+    const int shape = a.prefill_shape != kPrefillAuto ? a.prefill_shape : prefill_wide_shape(a);
+    if (shape != kPrefillNarrow) return launch_prefill_wide(a, shape, s);
     const bool gate_up = a.p[0].w2.qw != nullptr;
     const uint32_t gps = a.ksplit > 1 ? a.groups_per_split : a.k / 64;
     if (tuning().prefill_kernel == 2 || a.k % 128 != 0 || gps % 2 != 0) {  // 64 columns per step
@@ -747,8 +742,6 @@ hipError_t launch_prefill(MfmaArgs &a, hipStream_t s) {
     }
     if (gate_up) return launch_prefill_shape<8, 2, 4, 2, 2, 1, 2>(a, s);
     if (a.ksplit > 1) return launch_prefill_shape<8, 2, 4, 1, 2, 1, 2>(a, s);
-    // Few tiles (more of them take the wide kernel): two groups of waves per tile split its steps
-    // (qkv 20.2 -> 19.0 us; four groups: 21.8 us).
     return launch_prefill_shape<4, 1, 4, 1, 2, 1, 2, 2>(a, s);
 }
 

@@ -30,6 +30,7 @@
 #include <type_traits>
 
 #include "kr_internal.hpp"
+#include "launch_rules.hpp"
 #include "q4_prefill.hpp"
 
 namespace kr {
@@ -425,53 +426,26 @@ hipError_t launch_wide(MfmaArgs &a, hipStream_t s) {
     return a.xh ? launch_wide_shape<MF, NF, 1, false, OCC>(a, s) : launch_wide_shape<MF, NF, 1, true, OCC>(a, s);
 }
 
-// Tiles of rows x cols outputs over all problems.
-uint32_t tiles_of(const MfmaArgs &a, uint32_t rows, uint32_t cols) {
-    uint32_t t = 0;
-    for (int i = 0; i < a.np; ++i) t += ((a.m + rows - 1) / rows) * ((a.p[i].w.n + cols - 1) / cols);
-    return t;
-}
-
-// True when `tiles` give at least quarters / 4 blocks per compute unit.
-bool fills(uint32_t tiles, uint32_t quarters) { return tiles * 4 >= quarters * (uint32_t)device_cus(); }
-
 }  // namespace
 
-// About 1.25 blocks per CU at the most splits: below (kr_q4_mlp at m = 512, 32 tiles in 8 splits: 32.9 us and
-// 6.8 for the reduction) q4_prefill.hip's 4 splits of 128 x 128 tiles are as fast (37 + 5.3) with half the
-// partials; at m = 640 (40 tiles) the whole MLP takes 115 us against 125, at m = 1024 164 against 177.
-uint32_t prefill_wide_split(const MfmaArgs &a, uint32_t max_split) {
-    if (tuning().prefill_kernel != 0 || a.k % 128 != 0 || a.np != 1 || a.p[0].w2.qw) return 0;
-    const uint32_t groups = a.k / 64, tiles = tiles_of(a, 128, 256);
-    uint32_t split = 1;
-    while (split < max_split && !fills(tiles * split, 5) && groups / (split * 2) >= 8) split *= 2;
-    return fills(tiles * split, 5) ? split : 0;
-}
-
-// The widest shape that has enough tiles, else q4_prefill.hip.  Measured, us (this kernel / that one):
-//   gate/up pairs [2 x 11008, 2048], 128 x 128 tiles: in kr_q4_mlp (the whole call) m = 512 (344 tiles) 103 /
-//   100, 640 (430) 115 / 125, 1024 164 / 177, 3907 503 / 845;
-//   plain [12288, 4096]: 128 x 256 tiles at m = 512 (192) 73 / 104, at m = 256 (96) 68 / 55, where 64 x 256
-//   tiles (192) take 48; 64 x 128 tiles at m = 128 (192) 33 / 34;
-//   three projections [2048 + 256 + 256, 2048], m = 512: 64 x 128 tiles (160) 21.9 / 20.5.
+// Gate/up: 128 x 128 tiles (64 pairs) once they give 1.5 blocks per compute unit, else q4_prefill.hip's of the same
+// size: in kr_q4_mlp (the whole call, us, this kernel / that one) [2 x 11008, 2048] at m = 512 (344 tiles) 103 / 100, 640
+// (430) 115 / 125, 1024 164 / 177, 3907 503 / 845.  Plain projections: launch_rules.hpp.  (The same rule with and
+// without converted operands: KR_OPT_PREFILL_OPERANDS must not change the bits.)
 int prefill_wide_shape(const MfmaArgs &a) {
-    const uint32_t gps = a.ksplit > 1 ? a.groups_per_split : a.k / 64;
-    if (tuning().prefill_kernel != 0 || a.k % 128 != 0 || gps % 2 != 0) return 0;
-    // (the same rule with and without converted operands: KR_OPT_PREFILL_OPERANDS must not change the bits)
-    if (a.p[0].w2.qw) return fills(tiles_of(a, 128, 128), 6) ? 42 : 0;
-    const uint32_t tiles = tiles_of(a, 128, 256);
-    if (a.ksplit > 1) return fills(tiles * a.ksplit, 5) ? 42 : 0;
-    if (fills(tiles, 3)) return 42;
-    if (fills(tiles_of(a, 64, 256), 3)) return 22;
-    if (fills(tiles_of(a, 64, 128), 3)) return 21;
-    return 0;
+    if (tuning().prefill_kernel != 0 || a.k % 128 != 0 || a.ksplit > 1) return kPrefillNarrow;
+    uint32_t ns[kMaxMfmaProblems];
+    for (int i = 0; i < a.np; ++i) ns[i] = a.p[i].w.n;
+    if (a.p[0].w2.qw)
+        return prefill_tiles(a.m, ns, 1, 128, 128) * 4 >= 6 * (uint64_t)device_cus() ? kPrefillWide42 : kPrefillNarrow;
+    return prefill_choice(a.m, ns, a.np, a.k, 1, false, (uint32_t)device_cus()).shape;
 }
 
 hipError_t launch_prefill_wide(MfmaArgs &a, int shape, hipStream_t s) {
     switch (shape) {
-        case 42: return launch_wide<4, 2, 2>(a, s);
-        case 22: return launch_wide_shape<2, 2, 1, true, 2>(a, s);
-        case 21: return launch_wide_shape<2, 1, 1, true, 4>(a, s);
+        case kPrefillWide42: return launch_wide<4, 2, 2>(a, s);
+        case kPrefillWide22: return launch_wide_shape<2, 2, 1, true, 2>(a, s);
+        case kPrefillWide21: return launch_wide_shape<2, 1, 1, true, 4>(a, s);
         default: return hipErrorInvalidValue;
     }
 }
