@@ -116,7 +116,9 @@ const char *kr_last_error(void);
                                          * own X slices.  Bitwise the same results either way. */
 #define KR_OPT_SKINNY_GROUPS 15         /* few-token kernel, 17 <= m <= 63: 2 (default) 32-row launches, each
                                          * multiplying every unpacked weight word with two 16-row groups
-                                         * of x; 1 16-row launches.  Bitwise the same results either way. */
+                                         * of x (over a long K without a workspace: where estimated faster
+                                         * than one group on more blocks); 1 16-row launches or blocks.
+                                         * Bitwise the same results either way. */
 #define KR_OPT_SKINNY_DEPTH 16          /* few-token kernel, launches with no bias and no accumulation:
                                          * 0 (default) three register buffers of tile words (two tiles
                                          * in flight) when a block's run holds >= 6 tiles, else two;
@@ -193,8 +195,10 @@ int kr_q4_linear(const kr_q4_matrix *w, const uint16_t *x, uint32_t m,
  * same accumulate semantics) with a caller workspace.  The workspace lets
  * 5 <= m rows over a long K (more than 2048 columns, and at m >= 64 few
  * output tiles) split K over blocks into f32 partials, summed in a fixed
- * order.  kr_q4_linear has no such buffer: there a few tokens over a long row
- * take the token GEMV in chunks, and more take the unsplit tiled kernel.
+ * order.  kr_q4_linear has no such buffer: there up to 16 tokens over a long
+ * row (k <= 16384) take the token GEMV in chunks; up to 63 the few-token
+ * kernel walking all of K in each block, where that is estimated faster than
+ * the prefill kernel's unsplit tiles; and more take those.
  * Results are within f32 summation order of kr_q4_linear's, and the same
  * bits from run to run.
  * workspace: kr_q4_linear_workspace_bytes(m, w->n, w->k) bytes, 16-byte

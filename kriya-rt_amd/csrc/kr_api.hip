@@ -198,18 +198,10 @@ bool skinny_fits(uint32_t m, const Q4Mat &w, bool have_partial) {
     return m >= 2 && m <= kSkinnyChunkMaxM && skinny_supported(w) && (have_partial || skinny_ksplit(w.k) == 1);
 }
 
-// The same kernel over a K of several slabs without room for partials (its slab loop), `rows` weight rows in
-// all.  Before / with it, us: gate/up [2 x 9536, 3072], m = 2 .. 16 67-70 / 17, m = 32 41 / 22, m = 40 41 / 39;
-// q/k/v [4608, 3584], m = 2 45 / 10; linear [3584, 18944], m = 8 255 / 28, m = 32 77 / 39; [2048, 11008], m = 27
-// 46 / 18, m = 63 46 / 24; [16384, 2304], m = 24 16 / 20; [65536, 4096], m = 32 79 / 54.  So: gate/up up to 32
-// tokens; other launches up to 16 (kr_q4_linear: beyond k = 16384, the token GEMV's limit), and above where it is estimated faster (past 32 clearly so) than the prefill
-// kernels' 64-token tiles, whose time is about 4 us + 1.02 per 256 columns for every 16384 rows.
-bool skinny_loops(uint32_t m, const Q4Mat &w, uint32_t rows, bool gate_up) {
-    if (m < 2 || m > kSkinnyChunkMaxM || !skinny_supported(w) || skinny_ksplit(w.k) == 1) return false;
-    if (m <= (gate_up ? 32u : 16u)) return true;
-    if (gate_up) return false;
-    const float prefill = (4.0f + 0.004f * (float)w.k) * std::max(1.0f, (float)rows / 16384.0f);
-    return skinny_loop_us(m, rows, w.k, false) < (m <= 32 ? 1.0f : 0.8f) * prefill;
+// The same kernel over a K of several slabs without room for partials (its slab loop).
+bool skinny_loops(uint32_t m, const Q4Mat &w, const uint32_t *ns, int np, bool gate_up) {
+    return m >= 2 && m <= kSkinnyChunkMaxM && skinny_supported(w) && skinny_ksplit(w.k) > 1 &&
+           slab_loop_pays(m, ns, np, w.k, gate_up, (uint32_t)device_cus());
 }
 
 size_t partial_bytes(uint32_t m, uint32_t n, uint32_t k, int nw) {
@@ -498,7 +490,7 @@ int kr_q4_linear(const kr_q4_matrix *w, const uint16_t *x, uint32_t m, void *y, 
         }
         return ok();
     }
-    if (skinny_loops(m, a, w->n, false))
+    if (skinny_loops(m, a, &w->n, 1, false))
         return hip_status(run_skinny(a, nullptr, x, m, y, nullptr, w->n, y_dtype, accumulate, 0, nullptr, s),
                           "kr_q4_linear");
     MfmaArgs args = mfma_args(x, m, w->k, y_dtype, accumulate);
@@ -538,7 +530,7 @@ int kr_q4_gate_up_act(const kr_q4_matrix *gate, const kr_q4_matrix *up, const ui
         return hip_status(launch_gemv_tokens(g, &u, x, m, act_out, gate->n, epi, activation, nullptr, s),
                           "kr_q4_gate_up_act");
     }
-    if ((skinny_fits(m, g, false) || skinny_loops(m, g, gate->n, true)) && skinny_supported(u))
+    if ((skinny_fits(m, g, false) || skinny_loops(m, g, &gate->n, 1, true)) && skinny_supported(u))
         return hip_status(run_skinny(g, &u, x, m, act_out, nullptr, gate->n, act_dtype, 0, activation, nullptr, s),
                           "kr_q4_gate_up_act");
     MfmaArgs args = mfma_args(x, m, gate->k, act_dtype, 0);
@@ -580,7 +572,8 @@ int kr_q4_qkv(const kr_q4_matrix *q, const kr_q4_matrix *k, const kr_q4_matrix *
         }
         return ok();
     }
-    if ((skinny_fits(m, to_mat(q), false) || skinny_loops(m, to_mat(q), q->n + k->n + v->n, false)) && skinny_supported(to_mat(k)) &&
+    const uint32_t ns[3] = {q->n, k->n, v->n};
+    if ((skinny_fits(m, to_mat(q), false) || skinny_loops(m, to_mat(q), ns, 3, false)) && skinny_supported(to_mat(k)) &&
         skinny_supported(to_mat(v)))
         return hip_status(run_skinny_qkv(mats, biases, outs, x, m, out_dtype, nullptr, 0.0f, s), "kr_q4_qkv");
     MfmaArgs args = mfma_args(x, m, q->k, out_dtype, 0);

@@ -248,8 +248,6 @@ hipError_t launch_moe_combine(const float *d, const float *w, uint32_t T, uint32
                               int accumulate, hipStream_t s);
 // Number of K splits (blocks per N tile) the dense skinny launcher uses for rows of k columns.
 uint32_t skinny_ksplit(uint32_t k);
-// Estimated microseconds of the few-token kernel's slab loop (dense, K of several slabs, no partials).
-float skinny_loop_us(uint32_t m, uint32_t rows, uint32_t k, bool gate_up);
 // True when one block of the grouped kernel covers rows of k columns (no K split).
 bool skinny_grouped_fits(uint32_t k);
 // The few-token kernel needs k % 64 == 0, and 4-byte aligned scales/biases when k % 128 == 0

@@ -1,15 +1,17 @@
-// launch_rules.hpp — which prefill launch a shape takes: plain host arithmetic on sizes, no HIP (the tests compile it
-// with the host compiler).
+// launch_rules.hpp — which launch a shape takes: plain host arithmetic on sizes, no HIP (the tests compile it with the
+// host compiler).
 //
-// A launch's blocks run in rounds of one per compute unit, so its time is close to
+// Prefill launches.  A launch's blocks run in rounds of one per compute unit, so its time is close to
 //     fixed + rounds (round + step K / 128) + partial (f32 partials written and summed, in millions),
 // also past one resident block per unit: they share its matrix cores.  The constants are least-squares fits to launches
 // on MI355X (256 compute units) over copies of the weights in turn (none in an L2), captured in graphs: m = 17 .. 4096,
-// n = 256 .. 151936, K = 1024 .. 18944, 2913 unsplit calls and 2190 with room for partials, each in every shape; the
-// median error is 5 %.  Counting rounds is what decides: a tile half full of padding costs what a full one does.
+// n = 256 .. 151936, K = 1024 .. 18944, 2913 unsplit calls and 2190 with room for partials, each in every shape: half
+// of them lie within 4 %, nine in ten within 15 %.  Counting rounds is what decides: a tile half full of padding costs what a full one does.
 #pragma once
 
 #include <stdint.h>
+
+#include <algorithm>
 
 namespace kr {
 
@@ -92,6 +94,58 @@ inline PrefillChoice prefill_choice(uint32_t m, const uint32_t *ns, int np, uint
     }
     for (uint32_t split = 2; split <= max_split && k / 64 / split >= 8; split *= 2) consider(kCostWideSplit, split, 1.0f);
     return best;
+}
+
+// ---- the few-token kernel's slab loop (q4_skinny.hip): K of several slabs, no room for partials
+constexpr uint32_t kSlabColumns = 2048;      // K columns per slab
+constexpr uint32_t kSlabLoopBlocks = 256;    // KR_OPT_SKINNY_MAX_BLOCKS' default
+
+// Estimated microseconds over `tiles` weight tiles (16 rows; gate/up 8 pairs) in groups of 16 mg token rows, at most
+// `blocks` blocks: per slab, the staging of X and the block's tiles.  Fitted to 2160 calls as above, m = 17 .. 63, n =
+// 256 .. 49152, K = 2112 .. 18944 (nine in ten within 12 %).  One or two rows in the last group take up to 25 % longer
+// over a long run of tiles (n = 65536, K = 3072: 61.9 us at m = 17, 51.5 at m = 20).
+inline float slab_loop_us(uint32_t m, uint32_t tiles, uint32_t k, uint32_t mg, uint32_t blocks) {
+    const uint32_t groups = (m + 16 * mg - 1) / (16 * mg), cap = std::max<uint32_t>(1, blocks / groups);
+    const float per = (float)((tiles + cap - 1) / cap), slabs = (float)((k + kSlabColumns - 1) / kSlabColumns);
+    const float us = mg == 1 ? 2.4f + slabs * (1.6f + 1.43f * per) : 2.2f + slabs * (3.75f + 1.42f * per);
+    return (m % 16 == 1 || m % 16 == 2) && m > 16 && per > 4.0f ? 1.15f * us : us;
+}
+
+// Groups of 16 token rows per block: one, on more blocks, while there are few tiles, else two per unpacked word.
+// options: KR_OPT_SKINNY_GROUPS and KR_OPT_SKINNY_MAX_BLOCKS (the same bits under any).
+inline uint32_t slab_loop_groups(uint32_t m, uint32_t tiles, uint32_t k, uint32_t groups_option, uint32_t blocks) {
+    return m > 16 && groups_option != 1 && slab_loop_us(m, tiles, k, 2, blocks) < slab_loop_us(m, tiles, k, 1, blocks) ? 2 : 1;
+}
+
+// Whether the slab loop takes m token rows over `rows` weight rows in all (ns[i] of np problems; gate/up: one).  Before /
+// with it, us: gate/up [2 x 9536, 3072], m = 2 .. 16 67-70 / 17, m = 32 41 / 22, m = 40 41 / 39; q/k/v [4608, 3584], m = 2
+// 45 / 10; linear [3584, 18944], m = 8 255 / 28, m = 32 77 / 39; [2048, 11008], m = 27 46 / 20, m = 63 46 / 27.  So: gate/up
+// up to 32 tokens; other launches up to 16, and above where it is estimated faster than the prefill launch these sizes
+// would take: [65536, 3072], m = 32 51.7 us against 38.3 there, [32768, 8192], m = 32 59.8 / 73.0; [6144, 4096], m = 33
+// 21.5 / 19.9; [2048, 2112] (an odd group count: 64-column steps), m = 33 11.5 / 18.5.  With one token tile no other
+// block reads a block's weights: about 0.06 us per MB over prefill_us.  13 of the 2160 calls come out 3 to 7 % slower than
+// on the prefill kernel, none more.  (Defaults on purpose, not the options: results must not depend on those.)
+inline bool slab_loop_pays(uint32_t m, const uint32_t *ns, int np, uint32_t k, bool gate_up, uint32_t cus) {
+    if (m <= (gate_up ? 32u : 16u)) return true;
+    if (gate_up) return false;
+    uint32_t tiles = 0, rows = 0;
+    for (int i = 0; i < np; ++i) {
+        tiles += (ns[i] + 15) / 16;
+        rows += ns[i];
+    }
+    float prefill;
+    if (k % 128 == 0) {
+        const int shape = prefill_choice(m, ns, np, k, 1, false, cus).shape;
+        prefill = prefill_us(kCostNarrow, m, ns, np, k, 1, cus);
+        for (const PrefillCost &w : kCostWide)
+            if (w.shape == shape) prefill = prefill_us(w, m, ns, np, k, 1, cus);
+    } else {
+        const uint64_t rounds = (prefill_tiles(m, ns, np, 64, 64) + cus - 1) / cus;
+        prefill = 5.0f + 0.36f * (float)(rounds + 1) * (float)k / 128.0f;
+    }
+    prefill += 0.06e-6f * (float)rows * (float)k * 0.5f;
+    const float loop = std::min(slab_loop_us(m, tiles, k, 1, kSlabLoopBlocks), slab_loop_us(m, tiles, k, 2, kSlabLoopBlocks));
+    return loop < 0.95f * prefill;
 }
 
 }  // namespace kr

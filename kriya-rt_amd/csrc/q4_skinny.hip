@@ -54,6 +54,7 @@
 #include <type_traits>
 
 #include "kr_internal.hpp"
+#include "launch_rules.hpp"
 
 namespace kr {
 
@@ -62,6 +63,7 @@ namespace {
 constexpr int kSkinnyWaves = 8;
 constexpr int kSkinnyPieces = 2;                                // 128-column pieces per wave
 constexpr int kSlabCols = kSkinnyWaves * kSkinnyPieces * 128;  // K columns per block
+static_assert(kSlabCols == (int)kSlabColumns, "launch_rules.hpp counts slabs");
 constexpr uint32_t kLoopTiles = 16;                            // tiles a slab-loop block sums at a time
 
 __device__ __forceinline__ uint32_t opq_s(uint32_t v) {
@@ -917,15 +919,6 @@ hipError_t launch_loop(SkinnyArgs &a, uint32_t items, hipStream_t s) {
     return hipGetLastError();
 }
 
-// Estimated microseconds of a slab-loop launch over `tiles` weight tiles in groups of 16 mg rows: per slab, the
-// staging of X and the block's tiles (measured: n = 2048, K = 11008, 6 slabs: 16 rows 17.4 us, 32 rows 28.1;
-// gate/up [2 x 9536, 3072], 2 slabs of 5 tiles: 17.1 and 22.3).
-float loop_us(uint32_t m, uint32_t tiles, uint32_t k, uint32_t mg) {
-    const uint32_t groups = (m + 16 * mg - 1) / (16 * mg), cap = std::max<uint32_t>(1, 256 / groups);
-    const float per = (float)((tiles + cap - 1) / cap);
-    return (float)skinny_ksplit(k) * (mg == 1 ? 1.6f + 1.3f * per : 2.8f + 1.8f * per);
-}
-
 template <bool GU, bool G, int MG, bool P, bool O>
 hipError_t launch_t(SkinnyArgs &a, uint32_t items, hipStream_t s) {
     // blocks per slab: every CU busy, each block a contiguous run of ceil(items / nblk) tiles
@@ -995,8 +988,7 @@ hipError_t launch_skinny(SkinnyArgs &a, hipStream_t s) {
                        : launch_t<false, true, 1, false, false>(a, items, s);
     if (gate_up && pre) return hipErrorInvalidValue;  // gate/up launches have neither
     if (loop) {
-        // 16-row groups on more blocks while there are few tiles, else two groups per unpacked word
-        if (a.m > 16 && loop_us(a.m, items, a.k, 2) < loop_us(a.m, items, a.k, 1))
+        if (slab_loop_groups(a.m, items, a.k, (uint32_t)tuning().skinny_groups, (uint32_t)tuning().skinny_max_blocks) == 2)
             return gate_up ? launch_loop<true, 2>(a, items, s) : launch_loop<false, 2>(a, items, s);
         return gate_up ? launch_loop<true, 1>(a, items, s) : launch_loop<false, 1>(a, items, s);
     }
@@ -1009,11 +1001,6 @@ hipError_t launch_skinny(SkinnyArgs &a, hipStream_t s) {
 }
 
 uint32_t skinny_ksplit(uint32_t k) { return (k + kSlabCols - 1) / kSlabCols; }
-
-float skinny_loop_us(uint32_t m, uint32_t rows, uint32_t k, bool gate_up) {
-    const uint32_t tiles = (rows + (gate_up ? 7 : 15)) / (gate_up ? 8 : 16);
-    return m > 16 ? std::min(loop_us(m, tiles, k, 1), loop_us(m, tiles, k, 2)) : loop_us(m, tiles, k, 1);
-}
 
 bool skinny_grouped_fits(uint32_t k) { return k % 128 == 0 && skinny_ksplit(k) == 1; }  // even group counts only
 

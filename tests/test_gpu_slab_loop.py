@@ -68,6 +68,27 @@ def test_qkv(kq, m, k):
         assert_rms_close(outs[i].cpu().numpy(), want, rel=2e-5, what=f"problem {i}")
 
 
+@pytest.mark.parametrize("m,n,k", [(27, 2048, 4160), (63, 3000, 2176), (8, 500, 16448)])
+def test_options_keep_the_bits(kq, m, n, k):
+    """KR_OPT_SKINNY_GROUPS and KR_OPT_SKINNY_MAX_BLOCKS choose row groups and grid, not the route or the sums."""
+    case(f"slab loop options m={m} n={n} k={k}")
+    s = synth()
+    wq, x = s.q4_weight(n, k, 7250 + m), dev_bf16(s.bf16_normal((m, k), 7251 + m))
+    w = q4_dev(kq, wq)
+    groups, blocks = kq.get_option(15), kq.get_option(6)
+    got = {}
+    try:
+        for o in ((2, 256), (1, 256), (2, 64), (1, 40), (2, 1000)):
+            kq.set_option(15, o[0])
+            kq.set_option(6, o[1])
+            got[o] = kq.q4_linear(w, x, out_dtype=kq.DTYPE_F32).cpu().numpy().view(np.uint32)
+    finally:
+        kq.set_option(15, groups)
+        kq.set_option(6, blocks)
+    for o, y in got.items():
+        assert np.array_equal(y, got[2, 256]), o
+
+
 def beyond_range(x):
     """Rows 1 .. 5 of x get an infinity of either sign, a NaN, one column and three columns of 3e37 (31 times that
     overflows f32, times a weight of about 0.1 it does not)."""

@@ -17,6 +17,10 @@ extern "C" int choice(uint32_t m, const uint32_t *ns, int np, uint32_t k, uint32
     *split = c.ksplit;
     return c.shape;
 }
+extern "C" int loop_pays(uint32_t m, uint32_t n, uint32_t k) { return kr::slab_loop_pays(m, &n, 1, k, false, 256); }
+extern "C" uint32_t loop_groups(uint32_t m, uint32_t n, uint32_t k, uint32_t option, uint32_t blocks) {
+    return kr::slab_loop_groups(m, (n + 15) / 16, k, option, blocks);
+}
 """
 
 
@@ -108,3 +112,23 @@ def test_converted_operand_takes_128_token_tiles(rules):
 def test_problems_add_up(rules):
     """Three projections of one x count as one launch: the tiles of all of them."""
     assert choose(rules, 512, [2048, 256, 256], 2048) == choose(rules, 512, [2560], 2048)
+
+
+# m, n, k: the slab loop, the prefill launch these sizes take otherwise (us)
+LOOP = [
+    ((17, 65536, 3072), 61.9, 37.2), ((24, 65536, 3072), 51.2, 37.4), ((32, 49152, 3072), 41.3, 34.9), ((17, 49152, 3072), 48.6, 34.7),
+    ((27, 2048, 11008), 20.5, 46.0), ((63, 2048, 11008), 27.7, 46.0), ((17, 8192, 18944), 66.2, 81.0), ((20, 32768, 8192), 59.0, 77.4),
+    ((63, 32768, 8192), 95.9, 76.9), ((48, 49152, 8192), 167.4, 99.8), ((17, 3072, 2304), 10.3, 14.7), ((49, 2048, 2304), 10.6, 14.7),
+]
+
+
+@pytest.mark.parametrize("shape,loop,prefill", LOOP)
+def test_slab_loop_where_it_pays(rules, shape, loop, prefill):
+    assert bool(rules.loop_pays(*shape)) == (loop < prefill)
+
+
+def test_slab_loop_groups_follow_the_options(rules):
+    """KR_OPT_SKINNY_GROUPS = 1 keeps 16-row groups, and the choice is made for KR_OPT_SKINNY_MAX_BLOCKS' grid."""
+    assert rules.loop_groups(32, 65536, 3072, 2, 256) == 2 and rules.loop_groups(32, 65536, 3072, 1, 256) == 1
+    assert rules.loop_groups(16, 65536, 3072, 2, 256) == 1
+    assert rules.loop_groups(27, 2048, 11008, 2, 256) == 1 and rules.loop_groups(27, 2048, 11008, 2, 64) == 2
