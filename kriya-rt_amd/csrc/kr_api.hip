@@ -911,11 +911,8 @@ int run_moe_experts(const kr_q4_matrix *gate, const kr_q4_matrix *up, const kr_q
                           "kr_q4_moe_experts (combine)");
     }
 
-    // Ten tokens per expert (were they even): the grouped products, whose operands need the workspace's last part.
-    // Below, the few-token kernel's 16-row tiles move fewer zero rows: 60 experts, top 4, 64 tokens 104 us against 134,
-    // 128 tokens 135 / 140, 160 tokens 150 / 144, 256 tokens 185 / 153, 1000 tokens 480 / 222; 16 experts of [512,
-    // 1024], 60 tokens 42 / 30.
-    if (assign / std::min(experts, assign) >= 10 && workspace_bytes >= moe_grouped_bytes(tokens, topk, hidden, inter) &&
+    // the grouped products need the workspace's last part for their operands
+    if (moe_grouped_pays(assign, experts, hidden, inter) && workspace_bytes >= moe_grouped_bytes(tokens, topk, hidden, inter) &&
         grouped_fits(inter, hidden, tokens, experts, assign) && grouped_fits(hidden, inter, assign, experts, assign)) {
         uint16_t *xp = (uint16_t *)d;  // until the down projection writes d
         char *xsu = (char *)d + round_up((size_t)tokens * hidden * 2, 256);

@@ -148,4 +148,33 @@ inline bool slab_loop_pays(uint32_t m, const uint32_t *ns, int np, uint32_t k, b
     return loop < 0.95f * prefill;
 }
 
+// ---- routed experts (q4_grouped.hip, q4_skinny.hip, moe.hip); tokens per expert as if they were even
+
+// Grouped matrix products instead of the few-token kernel, which takes 16 tokens of an expert at a time and moves fewer
+// zero rows: from 8 to 10 tokens per expert where there are many experts (one of them has 17 by then; the later the larger
+// their matrices), later still where few experts leave compute units idle.  Measured crossings (random routing, tokens
+// per expert): 60 experts [1408, 2048] 10, 32 11, 16 13, 8 15, 4 25, 2 40; 16 [2048, 2048] 12, 8 15, 4 28; 64 [768, 2048] 9,
+// 32 9, 16 10, 8 14, 4 26; 32 [512, 1024] below 8, 16 8, 8 13, 4 24, 2 28.  The rule: 10.9, 11.8, 13.5, 17, 24, 38; 13.5, 17, 24;
+// 8.9, 9.8, 11.5, 15, 22; 9.8, 11.5, 15, 22, 36.
+inline bool moe_grouped_pays(uint32_t assign, uint32_t experts, uint32_t hidden, uint32_t inter) {
+    return assign >= ((uint64_t)hidden * inter >= 2500000 ? 10u : 8u) * (uint64_t)experts + 56;
+}
+
+// 96-token tiles instead of 32-token ones, ntiles of them side by side per expert: once they hold a second fragment on
+// average (the third is skipped where there are no tokens), if they still give two blocks per three compute units (down:
+// or one per two, well filled).  This / 32-token tiles: gate/up of [1408, 2048], 60 experts 1.00 at 22 tokens per expert,
+// 0.96 at 28, 0.79 at 40; 8 (176 blocks) 1.03 at 28, 0.89 at 40; 4 (88) 1.15 at 64, 0.97 at 128 (176); [2048, 2048], 8 (256)
+// 1.00 at 24, 0.90 at 28; down: 60 experts 1.00 at 20, 0.93 at 32; 16 (256) 0.91 at 28; 8 (128) 1.04 at 40, 0.97 at 64.
+inline bool moe_wide_tiles(uint32_t assign, uint32_t experts, uint32_t ntiles, bool gate_up, uint32_t cus) {
+    const uint32_t e = std::max(1u, std::min(experts, assign)), per = assign / e;
+    const uint64_t blocks = (uint64_t)e * ((per + 95) / 96) * ntiles;
+    if (!gate_up && per > 56 && blocks * 2 >= cus) return true;
+    return per > (gate_up ? 23u : 20u) && blocks * 3 >= 2 * (uint64_t)cus;
+}
+
+// Slots of the sorted list in parts, one per wave (3.6 us plus 0.6 per 1000 assignments), instead of a pass over all
+// assignments for every sixteen experts (3.0 us plus 1.2 per 1000 and sixteen): 8 experts, 256 assignments 3.65 / 3.35 us,
+// 512 3.79 / 3.87, 2048 5.2 / 7.2; 32 experts, 192 3.60 / 3.68; 60 experts, 128 3.60 / 3.88, 4096 6.8 / 35.6.
+inline bool moe_route_parts(uint32_t assign, uint32_t experts) { return (uint64_t)((experts + 15) / 16) * assign > 480; }
+
 }  // namespace kr

@@ -19,16 +19,15 @@
 #include <math.h>
 
 #include "kr_internal.hpp"
+#include "launch_rules.hpp"
 #include "moe_route.hpp"
 
 namespace kr {
 
-// More assignments than this take their slots in parts, one per wave.
-constexpr uint32_t kRouteChunked = 256;
-
 // One block.  logits != nullptr: route one token per wave (writes experts,
 // weights); else the assignments `experts` are given.  Then counts, offsets
-// and the sorted list.
+// and the sorted list.  kParts: moe_route_parts() (launch_rules.hpp).
+template <bool kParts>
 __global__ __launch_bounds__(1024) void moe_route_kernel(const float *logits, uint32_t T, uint32_t E, uint32_t K,
                                                          int normalize, uint32_t *experts, float *weights,
                                                          uint32_t *counts, uint32_t *offsets, uint32_t *sorted) {
@@ -104,7 +103,7 @@ __global__ __launch_bounds__(1024) void moe_route_kernel(const float *logits, ui
         if (e < E) counts[e] = s_cnt[e];
     }
     const uint64_t below = (1ull << lane) - 1ull;
-    if (total > kRouteChunked) {
+    if constexpr (kParts) {
         // Many assignments: wave w takes the w-th part of them, 64 at a time.  The waves' counts per expert give
         // each wave its first slot of every bucket; inside 64 assignments the lanes of one expert are found
         // by eight ballots, one per bit of the id.  (4000 assignments of 60 experts: 31 us with a pass over
@@ -197,8 +196,12 @@ hipError_t launch_moe_route(const float *logits, uint32_t T, uint32_t E, uint32_
         if (hipError_t e = hipGetLastError()) return e;
         logits = nullptr;
     }
-    hipLaunchKernelGGL(moe_route_kernel, dim3(1), dim3(1024), 0, s, logits, T, E, K, normalize, experts, weights,
-                       counts, offsets, sorted);
+    if (moe_route_parts(T * K, E))
+        hipLaunchKernelGGL(moe_route_kernel<true>, dim3(1), dim3(1024), 0, s, logits, T, E, K, normalize, experts, weights,
+                           counts, offsets, sorted);
+    else
+        hipLaunchKernelGGL(moe_route_kernel<false>, dim3(1), dim3(1024), 0, s, logits, T, E, K, normalize, experts, weights,
+                           counts, offsets, sorted);
     return hipGetLastError();
 }
 

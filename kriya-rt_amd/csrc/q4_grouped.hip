@@ -24,6 +24,7 @@
 #include <type_traits>
 
 #include "kr_internal.hpp"
+#include "launch_rules.hpp"
 #include "q4_prefill.hpp"
 
 namespace kr {
@@ -355,14 +356,14 @@ hipError_t launch_grouped_t(const GroupedArgs &a, hipStream_t s) {
     return hipGetLastError();
 }
 
-// 96-token tiles from about 20 tokens per expert (were they even), 32-token tiles (four blocks per CU) below:
-// 60 experts, hidden 2048, inter 1408, top 4, experts' calls in us with 32 / 64 / 96 / 128-token tiles: 256 tokens
-// 153 / 150 / - / 164, 400 tokens 175 / 170 / 168 / -, 1000 tokens 326 / 285 / 222 / 223; 8 experts, 2000 tokens, top 2:
-// 288 / 223 / 205 / 261 (128-token tiles spill).
+// 32-token tiles (four blocks per CU) or 96-token ones, by moe_wide_tiles() (launch_rules.hpp).  (8 experts, 2000 tokens, top
+// 2, the experts' call in us with 32 / 64 / 96 / 128-token tiles: 288 / 223 / 205 / 261; the last spill.)
 template <bool kGateUp>
 hipError_t launch_grouped_m(const GroupedArgs &a, hipStream_t s) {
-    if (a.assign / std::min(a.experts, a.assign) <= 20) return launch_grouped_t<1, kGateUp, 4>(a, s);
-    return launch_grouped_t<3, kGateUp, 2>(a, s);
+    constexpr uint32_t kCols = kGateUp ? 64 : 128;
+    if (moe_wide_tiles(a.assign, a.experts, (a.rows + kCols - 1) / kCols, kGateUp, (uint32_t)device_cus()))
+        return launch_grouped_t<3, kGateUp, 2>(a, s);
+    return launch_grouped_t<1, kGateUp, 4>(a, s);
 }
 
 }  // namespace

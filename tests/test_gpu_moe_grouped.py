@@ -74,6 +74,28 @@ def test_buckets(kq, counts, hidden, inter, act):
     assert_rms_close(z, y, what="few-token kernel")
 
 
+@pytest.mark.parametrize("pattern,times,hidden,inter", [
+    ((96, 97, 0, 95, 1, 64, 65, 193), 12, 256, 128),   # 96 experts: 96-token tiles in both launches; two steps, one step
+    ((40, 41, 0, 31, 33, 64, 97, 20), 8, 384, 640),    # three and five steps
+    ((40, 0, 129, 32, 7, 96, 3, 33), 3, 128, 1152),    # 24 experts: gate/up in 96-token tiles, down in 32-token ones
+])
+def test_wide_tiles(kq, pattern, times, hidden, inter):
+    """96-token tiles: enough experts that they fill two thirds of the compute units."""
+    counts = pattern * times
+    E = len(counts)
+    case(f"grouped experts, 96-token tiles E={E} hidden={hidden} inter={inter}")
+    ids = bucketed(counts, E)
+    (g, u, d), x, w, r = setup(kq, ids, E, hidden, inter, 6050)
+    want = O.moe_experts(O.Q4Planar(*g), O.Q4Planar(*u), O.Q4Planar(*d), E, x, ids, w, 0)
+    y = kq.moe_experts(q4_dev(kq, g), q4_dev(kq, u), q4_dev(kq, d), E, dev_bf16(x), r).cpu().numpy()
+    # An intermediate on a bf16 rounding boundary may round the other way, by 2^-7 of it at most: where one of 128 holds
+    # half of a token's 2-norm, 0.5 sqrt(128) / sqrt(128) * 2^-7 * |w| / rms(w) (up to 3 with these scales) = 1.2 % of the
+    # token's RMS.  Few do: 1e-3 in the 2-norm.
+    for t in range(ids.shape[0]):
+        assert_rms_close(y[t], want[t], rel=2e-2, what=f"token {t}")
+    assert np.linalg.norm(y - want) <= 1e-3 * np.linalg.norm(want)
+
+
 def test_topk_rows_and_determinism(kq):
     """Top-3 routing from logits (rows gathered through the sorted list), twice the same bits."""
     case("grouped experts T=70 E=8 K=3")

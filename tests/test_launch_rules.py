@@ -21,6 +21,13 @@ extern "C" int loop_pays(uint32_t m, uint32_t n, uint32_t k) { return kr::slab_l
 extern "C" uint32_t loop_groups(uint32_t m, uint32_t n, uint32_t k, uint32_t option, uint32_t blocks) {
     return kr::slab_loop_groups(m, (n + 15) / 16, k, option, blocks);
 }
+extern "C" int grouped_pays(uint32_t assign, uint32_t experts, uint32_t hidden, uint32_t inter) {
+    return kr::moe_grouped_pays(assign, experts, hidden, inter);
+}
+extern "C" int wide_tiles(uint32_t assign, uint32_t experts, uint32_t ntiles, int gate_up) {
+    return kr::moe_wide_tiles(assign, experts, ntiles, gate_up, 256);
+}
+extern "C" int route_parts(uint32_t assign, uint32_t experts) { return kr::moe_route_parts(assign, experts); }
 """
 
 
@@ -132,3 +139,42 @@ def test_slab_loop_groups_follow_the_options(rules):
     assert rules.loop_groups(32, 65536, 3072, 2, 256) == 2 and rules.loop_groups(32, 65536, 3072, 1, 256) == 1
     assert rules.loop_groups(16, 65536, 3072, 2, 256) == 1
     assert rules.loop_groups(27, 2048, 11008, 2, 256) == 1 and rules.loop_groups(27, 2048, 11008, 2, 64) == 2
+
+
+# experts, tokens per expert, hidden, inter: the few-token kernel's time over the grouped products' (the routed stage)
+GROUPED = [
+    ((8, 10, 2048, 1408), 0.82), ((8, 12, 2048, 1408), 0.86), ((8, 20, 2048, 1408), 1.18), ((4, 16, 2048, 1408), 0.85),
+    ((4, 20, 2048, 1408), 0.94), ((4, 32, 2048, 1408), 1.11), ((2, 32, 2048, 1408), 0.92), ((16, 10, 2048, 1408), 0.81),
+    ((16, 16, 2048, 1408), 1.2), ((60, 8, 2048, 1408), 0.80), ((60, 12, 2048, 1408), 1.08), ((32, 10, 2048, 1408), 0.82),
+    ((128, 8, 2048, 768), 0.95), ((128, 12, 2048, 768), 1.27), ((64, 10, 2048, 768), 1.24), ((16, 12, 1024, 512), 1.25),
+    ((32, 10, 1024, 512), 1.3), ((8, 16, 1024, 2048), 1.15), ((8, 10, 1024, 2048), 0.9), ((60, 10, 1152, 640), 1.45),
+]
+
+
+@pytest.mark.parametrize("routing,ratio", GROUPED)
+def test_grouped_products_where_they_pay(rules, routing, ratio):
+    experts, per, hidden, inter = routing
+    assert bool(rules.grouped_pays(experts * per, experts, hidden, inter)) == (ratio > 1)
+
+
+# experts, tokens per expert, tiles side by side, gate/up: the 96-token tiles' time over the 32-token tiles'
+TILES = [
+    ((4, 64, 22, 1), 1.15), ((8, 40, 22, 1), 0.89), ((8, 96, 8, 1), 1.18), ((32, 28, 8, 1), 0.93), ((16, 128, 8, 1), 0.92),
+    ((32, 20, 22, 1), 1.07), ((60, 40, 22, 1), 0.79), ((4, 256, 12, 1), 0.98), ((1, 160, 32, 1), 1.18), ((16, 28, 16, 0), 0.91),
+    ((8, 40, 16, 0), 1.04), ((4, 80, 16, 0), 1.11), ((60, 32, 16, 0), 0.93), ((8, 128, 16, 0), 0.91), ((2, 160, 16, 0), 1.10),
+    ((8, 28, 32, 1), 0.9), ((8, 64, 16, 0), 0.93), ((8, 25, 32, 1), 0.95),
+]
+
+
+@pytest.mark.parametrize("launch,ratio", TILES)
+def test_wide_tiles_where_they_pay(rules, launch, ratio):
+    experts, per, ntiles, gate_up = launch
+    wide = bool(rules.wide_tiles(experts * per, experts, ntiles, gate_up))
+    assert (ratio if wide else 1 / ratio) <= 1.04
+
+
+@pytest.mark.parametrize("experts,assign,passes,parts", [
+    (8, 256, 3.35, 3.65), (8, 320, 3.48, 3.71), (4, 384, 3.67, 3.77), (8, 1024, 4.92, 4.15), (16, 768, 4.52, 3.93), (32, 512, 5.03, 3.74),
+    (60, 256, 4.92, 3.63), (128, 128, 4.87, 3.63), (256, 65, 5.75, 3.72), (16, 128, 3.09, 3.62)])
+def test_route_parts_where_they_pay(rules, experts, assign, passes, parts):
+    assert bool(rules.route_parts(assign, experts)) == (parts < passes)
