@@ -5,8 +5,9 @@
 //     fixed + rounds (round + step K / 128) + partial (f32 partials written and summed, in millions),
 // also past one resident block per unit: they share its matrix cores.  The constants are least-squares fits to launches
 // on MI355X (256 compute units) over copies of the weights in turn (none in an L2), captured in graphs: m = 17 .. 4096,
-// n = 256 .. 151936, K = 1024 .. 18944, 2913 unsplit calls and 2190 with room for partials, each in every shape: half
-// of them lie within 4 %, nine in ten within 15 %.  Counting rounds is what decides: a tile half full of padding costs what a full one does.
+// n = 256 .. 151936, K = 128 .. 18944, 4485 unsplit calls and 2190 with room for partials, each in every shape: half of
+// them lie within 5 %, nine in ten within 17 %.  Counting rounds is what decides: a tile half full of padding costs what
+// a full one does.
 #pragma once
 
 #include <stdint.h>
@@ -29,12 +30,12 @@ struct PrefillCost {
     uint32_t rows, cols;
     float fixed, round, step, partial;
 };
-constexpr PrefillCost kCostNarrow = {kPrefillNarrow, 64, 64, 5.3f, 0.3f, 0.45f, 0.0f};
-constexpr PrefillCost kCostNarrowSplit = {kPrefillNarrow, 128, 128, 16.2f, -5.4f, 1.17f, 2.03f};
-constexpr PrefillCost kCostWide[3] = {{kPrefillWide42, 128, 256, 3.2f, 4.5f, 1.64f, 0.0f},
-                                      {kPrefillWide22, 64, 256, 5.4f, 0.1f, 1.13f, 0.0f},
-                                      {kPrefillWide21, 64, 128, 8.7f, -3.3f, 0.83f, 0.0f}};
-constexpr PrefillCost kCostWideSplit = {kPrefillWide42, 128, 256, 12.9f, -3.7f, 1.67f, 1.74f};
+constexpr PrefillCost kCostNarrow = {kPrefillNarrow, 64, 64, 3.6f, 2.2f, 0.41f, 0.0f};
+constexpr PrefillCost kCostNarrowSplit = {kPrefillNarrow, 128, 128, 12.3f, 0.0f, 1.09f, 1.26f};
+constexpr PrefillCost kCostWide[3] = {{kPrefillWide42, 128, 256, 4.3f, 4.0f, 1.62f, 0.0f},
+                                      {kPrefillWide22, 64, 256, 4.3f, 1.5f, 1.1f, 0.0f},
+                                      {kPrefillWide21, 64, 128, 4.1f, 0.7f, 0.64f, 0.0f}};
+constexpr PrefillCost kCostWideSplit = {kPrefillWide42, 128, 256, 9.9f, 0.0f, 1.66f, 1.41f};
 // A wide shape has to be this much faster by estimate: at 0.93 one of those calls comes out more than 3 % slower
 // than on the narrow kernel (by 5 %).
 constexpr float kWideMargin = 0.93f;
@@ -84,12 +85,15 @@ inline PrefillChoice prefill_choice(uint32_t m, const uint32_t *ns, int np, uint
     for (const PrefillCost &c : kCostWide) {
         float scale = 1.0f;
         if (converted && c.shape != kPrefillWide42) continue;
-        // One round of 64 x 128 tiles has fewer loads in flight than two of 64 x 64: 16.0 / 17.3 us at K = 1536, but
-        // 18.9 / 18.0 at K = 2048, 35.5 / 33.3 at K = 4096 and 90 / 78 at 11008 (m = 2048, n = 1024, K = 4096: 36.5 /
-        // 41.4, but 33 with K split).
-        if (c.shape == kPrefillWide21 && prefill_tiles(m, ns, np, c.rows, c.cols) <= cus && k > 1536 &&
-            (m < 2048 || max_split > 1))
-            scale = 1.25f;
+        // One round of 64 x 128 tiles has fewer loads in flight than two of 64 x 64, which shows on long rows, rows a
+        // power of two apart and single token tiles: this / that, 15.7 / 17.4 us at K = 1536, 30.5 / 31.1 at 3584, but
+        // 15.0 / 14.3 at K = 1024 (the norm and [2048 + 512 + 512], m = 377), 18.9 / 18.0 at 2048, 35.5 / 33.3 at 4096, 90
+        // / 78 at 11008 and, m <= 64, 27.4 / 25.6 at 3072 (m = 2048, n = 1024, K = 4096: 36.5 / 41.4).  With room for
+        // partials a split is as good: 23.9 / 20.7 at K = 2816.
+        const bool one_round = prefill_tiles(m, ns, np, c.rows, c.cols) <= cus;
+        if (c.shape == kPrefillWide21 && one_round &&
+            ((k > 1536 && (max_split > 1 || m <= 64)) || (m < 2048 && (k % 1024 == 0 || k > 3584))))
+            scale = 1.5f;
         consider(c, 1, scale);
     }
     for (uint32_t split = 2; split <= max_split && k / 64 / split >= 8; split *= 2) consider(kCostWideSplit, split, 1.0f);
@@ -123,7 +127,7 @@ inline uint32_t slab_loop_groups(uint32_t m, uint32_t tiles, uint32_t k, uint32_
 // up to 32 tokens; other launches up to 16, and above where it is estimated faster than the prefill launch these sizes
 // would take: [65536, 3072], m = 32 51.7 us against 38.3 there, [32768, 8192], m = 32 59.8 / 73.0; [6144, 4096], m = 33
 // 21.5 / 19.9; [2048, 2112] (an odd group count: 64-column steps), m = 33 11.5 / 18.5.  With one token tile no other
-// block reads a block's weights: about 0.06 us per MB over prefill_us.  13 of the 2160 calls come out 3 to 7 % slower than
+// block reads a block's weights: about 0.05 us per MB over prefill_us.  13 of the 2160 calls come out 3 to 7 % slower than
 // on the prefill kernel, none more.  (Defaults on purpose, not the options: results must not depend on those.)
 inline bool slab_loop_pays(uint32_t m, const uint32_t *ns, int np, uint32_t k, bool gate_up, uint32_t cus) {
     if (m <= (gate_up ? 32u : 16u)) return true;
@@ -143,9 +147,9 @@ inline bool slab_loop_pays(uint32_t m, const uint32_t *ns, int np, uint32_t k, b
         const uint64_t rounds = (prefill_tiles(m, ns, np, 64, 64) + cus - 1) / cus;
         prefill = 5.0f + 0.36f * (float)(rounds + 1) * (float)k / 128.0f;
     }
-    prefill += 0.06e-6f * (float)rows * (float)k * 0.5f;
+    prefill += 0.05e-6f * (float)rows * (float)k * 0.5f;
     const float loop = std::min(slab_loop_us(m, tiles, k, 1, kSlabLoopBlocks), slab_loop_us(m, tiles, k, 2, kSlabLoopBlocks));
-    return loop < 0.95f * prefill;
+    return loop < 0.99f * prefill;
 }
 
 // ---- routed experts (q4_grouped.hip, q4_skinny.hip, moe.hip); tokens per expert as if they were even

@@ -68,16 +68,22 @@ UNSPLIT = [
     ((1500, 4096, 3584), 87.9, (62.1, 65.3, 65.3)),
     ((448, 16384, 1536), 44.3, (33.1, 32.0, 35.8)),
     ((2048, 1024, 4096), 41.4, (64.0, 44.3, 36.5)),
+    ((100, 2048, 256), 6.4, (10.7, 7.5, 5.6)),
+    ((193, 512, 768), 7.4, (17.5, 11.5, 8.4)),
+    ((640, 32000, 512), 73.7, (35.7, 33.4, 36.4)),
+    ((100, 16384, 128), 9.0, (9.9, 7.3, 5.6)),
+    ((256, 65536, 256), 57.4, (20.5, 20.5, 21.2)),
+    ((256, 1024, 768), 8.1, (17.9, 12.1, 9.8)),
 ]
 
 
-@pytest.mark.parametrize("shape,narrow,wide", UNSPLIT)
-def test_unsplit(rules, shape, narrow, wide):
+@pytest.mark.parametrize("shape,narrow,others", UNSPLIT)
+def test_unsplit(rules, shape, narrow, others):
     m, n, k = shape
     s, split = choose(rules, m, [n], k)
     assert split == 1
-    t = narrow if s == NARROW else wide[WIDE[s]]
-    assert t <= 1.04 * narrow and t <= 1.25 * min(narrow, *wide), (s, t)
+    t = narrow if s == NARROW else others[WIDE[s]]
+    assert t <= 1.04 * narrow and t <= 1.25 * min(narrow, *others), (s, t)
 
 
 # m, n, k: narrow (its own split); the three wide shapes unsplit; 128 x 256 tiles in 2, 4, 8 K parts (us; 0: too short)
@@ -99,12 +105,12 @@ SPLIT = [
 ]
 
 
-@pytest.mark.parametrize("shape,narrow,wide,parts", SPLIT)
-def test_with_room_for_partials(rules, shape, narrow, wide, parts):
+@pytest.mark.parametrize("shape,narrow,others,parts", SPLIT)
+def test_with_room_for_partials(rules, shape, narrow, others, parts):
     m, n, k = shape
     s, split = choose(rules, m, [n], k, max_split=8)
-    t = narrow if s == NARROW else wide[WIDE[s]] if split == 1 else parts[{2: 0, 4: 1, 8: 2}[split]]
-    best = min(v for v in (narrow, *wide, *parts) if v)
+    t = narrow if s == NARROW else others[WIDE[s]] if split == 1 else parts[{2: 0, 4: 1, 8: 2}[split]]
+    best = min(v for v in (narrow, *others, *parts) if v)
     assert 0 < t <= 1.04 * narrow and t <= 1.25 * best, (s, split, t)
 
 
