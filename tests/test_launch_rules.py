@@ -9,6 +9,8 @@ import subprocess
 
 import pytest
 
+import test_gpu_prefill_wide as wide
+
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "kriya-rt_amd", "csrc")
 SOURCE = """
 #include "launch_rules.hpp"
@@ -120,6 +122,15 @@ def test_converted_operand_takes_128_token_tiles(rules):
         for n, k in ((1024, 2816), (2048, 11008), (3584, 18944)):
             s, split = choose(rules, m, [n], k, max_split=8, converted=1)
             assert s in (NARROW, 42) and k // 64 // split >= 8
+
+
+def test_gpu_tests_reach_the_wide_launches(rules):
+    for (m, n, k), launch in wide.PLAIN_42:
+        assert choose(rules, m, [n], k) == launch
+    for (m, n, k), launch in wide.SPLIT_42:
+        assert choose(rules, m, [n], k, max_split=8) == launch
+    for (m, hidden, inter), launch in wide.MLP_DOWN:
+        assert choose(rules, m, [hidden], inter, max_split=8, converted=1) == launch
 
 
 def test_problems_add_up(rules):
