@@ -67,6 +67,101 @@ __device__ __forceinline__ void exact8(const Q4Mat &w, uint32_t n, const uint16_
         if (!__builtin_isfinite(src[e])) src[e] = sum[e];
 }
 
+// 16-byte epilogue accesses: the launch's outputs (or partials) and bias allow them.
+template <int EPI>
+__device__ __forceinline__ bool prefill_vec_out(const MfmaArgs &args, const MfmaProblem &P) {
+    if (EPI == kMfmaPartial) return (uintptr_t)args.partial % 16 == 0 && P.w.n % 8 == 0;
+    return (uintptr_t)P.out % 16 == 0 && P.ldo % 8 == 0 && (!P.bias || (uintptr_t)P.bias % 16 == 0);
+}
+
+// Eight consecutive output columns n .. n + 7 of token row m from LDS (src, 16-byte aligned, the activation
+// applied): bias, accumulation and the store, in 16-byte pieces when `vec`.  Columns beyond N are dropped.
+template <int EPI, bool kGateUp>
+__device__ __forceinline__ void prefill_store8(const MfmaArgs &args, const MfmaProblem &P, uint32_t ks, uint32_t m,
+                                               uint32_t n, float *src, bool vec) {
+    const uint32_t N = P.w.n;
+    const bool full = vec && n + 8 <= N;
+    if (kGateUp && args.act != 0) {  // rolled: the tanh of eight columns is long code
+#pragma unroll 1
+        for (int e = 0; e < 8; ++e) src[e] = activation(src[e], args.act) * src[32 + e];
+    }
+    f32x4 lo = reinterpret_cast<const f32x4 *>(src)[0], hi = reinterpret_cast<const f32x4 *>(src)[1];
+    if (kGateUp && args.act == 0) {
+        const f32x4 ul = reinterpret_cast<const f32x4 *>(src)[8], uh = reinterpret_cast<const f32x4 *>(src)[9];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            lo[e] = activation(lo[e], 0) * ul[e];
+            hi[e] = activation(hi[e], 0) * uh[e];
+        }
+        if (!full) {
+            reinterpret_cast<f32x4 *>(src)[0] = lo;
+            reinterpret_cast<f32x4 *>(src)[1] = hi;
+        }
+    }
+    if constexpr (EPI == kMfmaPartial) {
+        static_assert(!kGateUp, "partials of one matrix");
+        float *dst = args.partial + ((size_t)ks * args.m + m) * (size_t)N + n;
+        if (full) {
+            reinterpret_cast<f32x4 *>(dst)[0] = lo;
+            reinterpret_cast<f32x4 *>(dst)[1] = hi;
+        } else {
+#pragma unroll 1
+            for (uint32_t e = 0; e < 8 && n + e < N; ++e) dst[e] = src[e];
+        }
+        return;
+    }
+    const size_t o = (size_t)m * P.ldo + n;
+    if (full) {
+        auto add_bf16 = [&](u32x4 b) {
+            const uint32_t bb[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                f32x4 &t = e < 2 ? lo : hi;
+                t[2 * (e & 1)] += bf16_to_f32(bb[e] & 0xFFFFu);
+                t[2 * (e & 1) + 1] += bf16_to_f32(bb[e] >> 16);
+            }
+        };
+        if (P.bias) add_bf16(*reinterpret_cast<const u32x4 *>(P.bias + n));
+        if (args.out_f32) {
+            f32x4 *out = reinterpret_cast<f32x4 *>(reinterpret_cast<float *>(P.out) + o);
+            if (args.accumulate) {
+                lo += out[0];
+                hi += out[1];
+            }
+            out[0] = lo;
+            out[1] = hi;
+        } else {
+            u32x4 *out = reinterpret_cast<u32x4 *>(reinterpret_cast<uint16_t *>(P.out) + o);
+            if (args.accumulate) add_bf16(out[0]);
+            const u32x4 pk = {pack_bf16_rne(lo[0], lo[1]), pack_bf16_rne(lo[2], lo[3]), pack_bf16_rne(hi[0], hi[1]),
+                              pack_bf16_rne(hi[2], hi[3])};
+            out[0] = pk;
+            if (kGateUp && args.out_h)  // the same 8 values as the next projection's fp16 operand
+                *reinterpret_cast<u32x4 *>(args.out_h + o) = x_unit_f16(pk);
+        }
+        return;
+    }
+    // column by column from the LDS tile (a run-time index into registers would be moves), rolled: tails only
+#pragma unroll 1
+    for (uint32_t e = 0; e < 8 && n + e < N; ++e) {
+        float x = src[e];
+        if (P.bias) x += bf16_to_f32(P.bias[n + e]);
+        if (args.out_f32) {
+            float *out = reinterpret_cast<float *>(P.out);
+            out[o + e] = args.accumulate ? out[o + e] + x : x;
+        } else {
+            uint16_t *out = reinterpret_cast<uint16_t *>(P.out);
+            const uint32_t b = f32_to_bf16(args.accumulate ? x + bf16_to_f32(out[o + e]) : x);
+            out[o + e] = (uint16_t)b;
+            if (kGateUp && args.out_h) {  // element e of its 8-column unit goes to 2 (e % 4) + e / 4
+                const _Float16 hv = (_Float16)bf16_to_f32(b);
+                const uint32_t c = n + e;
+                args.out_h[o - n + (c & ~7u) + 2 * (c & 3u) + ((c & 7u) >> 2)] = __builtin_bit_cast(uint16_t, hv);
+            }
+        }
+    }
+}
+
 // MF x 32 token rows by 4 waves x NF x 32 weight rows per block.
 template <int MF, int NF, int NW>
 struct WideTile {
