@@ -20,8 +20,14 @@
  *   - Results do not depend on the launch grid: every output element is
  *     reduced by one wavefront in a fixed order (no atomics on data).
  *   - Activation range.  For m < 64 token rows (the GEMV and few-token
- *     kernels) every bf16 x is multiplied exactly (bf16 products, f32 sums).
- *     For m >= 64 (the prefill kernel) x is staged in fp16, as the reference's
+ *     kernels) every bf16 x is multiplied exactly (bf16 products, f32 sums),
+ *     up to |x| of about 1e36: x times an integer of up to 143 is summed in
+ *     f32, so beyond that, or with an infinite x, a sum can come out infinite
+ *     or NaN where x . w is not.  The launches that walk K inside their
+ *     blocks (k > 2048 without a workspace) and the grouped products of
+ *     prefill-sized MoE routings compute such outputs again in plain f32.
+ *     For m >= 64 (the prefill kernels; also 17 <= m <= 63 over k > 2048
+ *     without a workspace, where they are faster) x is staged in fp16, as the reference's
  *     M >= 64 kernels stage half (q4_gemm_and_moe.metal:2722-2724): exact for
  *     |x| in [2^-14, 65504]; outputs whose sums overflow fp16 are recomputed in
  *     f32 (exact), and values below 2^-14 keep fp16's subnormal precision
@@ -93,8 +99,10 @@ const char *kr_last_error(void);
 #define KR_OPT_GEMV_PERSISTENT_BLOCKS 5 /* grid of the persistent wave kernel (1024)       */
 #define KR_OPT_SKINNY_MAX_BLOCKS 6      /* grid cap of the few-token kernel (256; grouped
                                            MoE launches take twice this)                  */
-#define KR_OPT_PREFILL_KERNEL 7         /* m > 16: 0 register-dequant (default), 1 tiled, 2 register-dequant
-                                           with 64-column steps (0 takes 128 where k allows) */
+#define KR_OPT_PREFILL_KERNEL 7         /* m > 16: 0 (default) register-dequant, on 32x32x16 matrix instructions
+                                           where estimated faster, else on 16x16x32 with 128-column steps
+                                           where k allows; 1 tiled; 2 register-dequant on 16x16x32 with
+                                           64-column steps */
 #define KR_OPT_GEMV_LONG_ROWS 8         /* k > 4096 rows per long-row block: 4 (default), 8, 16; 0 split-K */
 #define KR_OPT_GEMV_TOKENS 9            /* 2 <= m <= 4: 1 (default) the GEMV kernels take all tokens per
                                            unpacked word (k <= 2048, or k <= 16384 without gate/up);
@@ -132,7 +140,8 @@ const char *kr_last_error(void);
 #define KR_OPT_PREFILL_XCD_SPLIT 19     /* prefill kernel with K split over blocks (kr_q4_mlp's down
                                          * projection at m >= 64): 1 (default) the blocks of each K split
                                          * are placed on their own XCDs, so that an L2 holds one K range
-                                         * of x; 0 the tile grouping of unsplit launches.  Bitwise the same. */
+                                         * of x; 0 the tile grouping of unsplit launches (on the 32x32x16
+                                         * kernel: each split's tiles over all XCDs).  Bitwise the same. */
 #define KR_OPT_ATTN_SLICE64 20          /* kr_rope_attention_decode with head_dim 128: slices of 64 positions
                                          * (one wave per 16 of them, all dims) instead of 16 (four waves
                                          * over the dims): 1 (default) when batch * kv_heads * slices still

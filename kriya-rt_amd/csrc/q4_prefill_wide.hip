@@ -1,7 +1,7 @@
 // q4_prefill_wide.hip — prefill Q4_G64 matmul with wide wave tiles on v_mfma_f32_32x32x16_f16.
 //
-// The same operation, operands and epilogues as q4_prefill.hip (which keeps the launches with few tiles and
-// the odd 64-group counts); replaces the reference's M >= 64 simdgroup kernels
+// The same operation, operands and epilogues as q4_prefill.hip (launch_rules.hpp says which of the two a launch
+// takes; odd 64-group counts stay there); replaces the reference's M >= 64 simdgroup kernels
 // (kernels/metal/q4_gemm_and_moe.metal:2708-3215) where there are enough tiles to fill the chip.
 //
 // What bounds it: instruction issue beside the matrix cores, and at large M the power limit.  A register
@@ -21,8 +21,11 @@
 //   * the epilogue passes 32 token rows at a time through a wave-private LDS tile (no block barriers; four
 //     consecutive columns per LDS write, eight per global store), and is kept short: unrolled tanh and
 //     per-element tails made it 11 us per block through the instruction cache, 5 us now.
-// Measured (K = 2048, 11008 gate/up pairs, m = 3907): 482 us on the 16x16x32 kernel, 321-333 here; the down
-// projection 2048 x 11008, 413 -> 180-194 us; [12288, 4096] at m = 512 / 2048 104 / 432 -> 73 / 204 us.
+// Measured (K = 2048, 11008 gate/up pairs, m = 3907): 482 us on the 16x16x32 kernel, 327 here (373 in the first ten
+// launches after idle, before the clock has settled); the down projection 2048 x 11008, 413 -> 174 us; [12288, 4096] at
+// m = 512 / 2048 88 / 425 -> 65 / 196 us.  Counters of these two launches: matrix cores busy 62 % and 50 % of SIMD cycles,
+// 5.6 and 4.7 VALU per matrix instruction (gate/up with the epilogue's), waves waiting to issue (SQ_WAIT_INST_ANY) 44 and
+// 26 % of their cycles and for memory or barriers (SQ_WAIT_ANY) 19 and 28 %, LDS bank conflicts 4 and 1 %.
 //
 // Column order: lane (c, h) of a 128-column step holds the 64 columns of group 2 g + h of weight row c (two
 // 16-byte loads); slice j multiplies word j of both halves, i.e. columns 64 h + 8 j .. + 7, so X is read

@@ -9,6 +9,7 @@ import subprocess
 
 import pytest
 
+import test_gpu_moe_grouped as grouped
 import test_gpu_prefill_wide as wide
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "kriya-rt_amd", "csrc")
@@ -188,6 +189,16 @@ def test_wide_tiles_where_they_pay(rules, launch, ratio):
     experts, per, ntiles, gate_up = launch
     wide = bool(rules.wide_tiles(experts * per, experts, ntiles, gate_up))
     assert (ratio if wide else 1 / ratio) <= 1.04
+
+
+def test_gpu_tests_reach_the_wide_tiles(rules):
+    down = []
+    for pattern, times, hidden, inter in grouped.WIDE_TILES:
+        experts, assign = len(pattern) * times, sum(pattern) * times
+        assert rules.grouped_pays(assign, experts, hidden, inter)
+        assert rules.wide_tiles(assign, experts, inter // 64, 1)
+        down.append(bool(rules.wide_tiles(assign, experts, -(-hidden // 128), 0)))
+    assert down == [True, True, False]
 
 
 @pytest.mark.parametrize("experts,assign,passes,parts", [
