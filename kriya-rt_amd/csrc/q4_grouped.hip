@@ -11,9 +11,10 @@
 // What bounds it: waiting.  At 1000 tokens x top 4 of 60 experts (hidden 2048, inter 1408) the counters of the gate/up
 // launch have the matrix cores busy 23 % of SIMD cycles, 10 VALU per matrix instruction and the waves, two per SIMD,
 // waiting 40 % of their cycles for memory and barriers (SQ_WAIT_ANY) and 30 % to issue (SQ_WAIT_INST_ANY; down: 21, 10,
-// 42, 32); it reads 320 MB for 198 MB of weights and x, a weight row once per expert and 96 tokens.  Per 128 columns and 32 x 32 outputs a wave issues 9 matrix instructions (288 cycles), 32
-// FMAs, and 56 VALU of unpacking shared by the row fragments.  The few-token kernel's 16-row chunks unpack and
-// sum across waves for every 16 tokens: 300 + 180 us there; here 121 + 63 us.
+// 42, 32); it reads 320 MB for 198 MB of weights and x, a weight row once per expert and 96 tokens.  Per 128 columns and
+// 32 x 32 outputs a wave issues 9 matrix instructions (288 cycles), 32 FMAs, and 56 VALU of unpacking shared by the row
+// fragments.  The few-token kernel's 16-row chunks unpack and sum across waves for every 16 tokens: 300 + 180 us there;
+// here 121 + 63 us.
 //
 // Operands.  X rows come with the columns of every 8 in the order the nibble pairs unpack in
 // (e0 e4 e1 e5 e2 e6 e3 e7) and one 16-byte unit (hi mid lo hi mid lo 0 0) of S per 64-column group:
